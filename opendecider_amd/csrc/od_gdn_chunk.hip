@@ -11,10 +11,11 @@
 // (the WY form of the chunked delta rule, as transformers' torch_chunk_gated_delta_rule evaluates it). Every
 // exponent is of a non-positive number, so nothing overflows whatever the decay.
 //
-// Two kernels. gdn_chunk_t, per (sequence, chunk, key head): K K^T on MFMA and T by forward substitution in fp32 for
+// gdn_chunk_t, per (sequence, chunk, key head): K K^T on MFMA and T by forward substitution in fp32 for
 // each value head of that key head, written as bf16 hi / lo in the layout the second kernel copies straight into
-// LDS, with the vectors gamma, e^gamma, e^{gamma_C - gamma} and e^{gamma_C}. gdn_chunk_state, per (sequence, value
-// head, 64 state columns), four waves of 16 columns each, chunk after chunk (the only sequential part): P from
+// LDS, with the vectors gamma, e^gamma, e^{gamma_C - gamma} and e^{gamma_C}. Then, chunk after chunk (the only
+// sequential part), gdn_chunk_roles (two or more chunks; a role per wave) or gdn_chunk_state (one chunk), both per
+// (sequence, value head, 64 state columns) with 16 columns per wave; gdn_chunk_state takes P from
 // K Q~^T on MFMA, then the products above. The state lives in the MFMA accumulators
 // (V_MFMA_F32_16X16X32_BF16, lane l: column l % 16, rows 4 (l / 16) + i of each 16 x 16 tile) and feeds the next
 // products straight from there: an accumulator tile's rows become a B operand's k-values in the order
@@ -457,6 +458,312 @@ __global__ __launch_bounds__(256) void gdn_chunk_state_kernel(CArgs p) {
   }
 }
 
+
+// ------------------------------------------------------------------------------------------------ gdn_chunk_roles
+// The chunk chain of a (sequence, value head, 64 columns) with a role per wave, so that the sequential part is only
+// the chunk's products:
+//   chain waves 0..3    16 state columns each: U = T V, X = K S_0 and Y = Q S_0 from one split of S_0,
+//                       delta = U - T (e^gamma X), the state update, O = e^gamma Y + P delta
+//   staging waves 4..7  chunk c + 2 from registers to LDS and the loads of chunk c + 4, P of chunk c + 1, the output
+//                       stores of chunk c - 1
+// Each role is a loop of its own (the registers of one role are not live in the other) with one barrier per chunk
+// over three stage buffers. Bound: the chain wave's own chunk, ~210 vector instructions, 64 MFMAs and ~45 LDS reads in
+// sequence, about 2500 cycles, with the staging waves just below it (4 x 4096 tokens, 32 heads: 2950 cycles a chunk
+// against 6500 with every wave doing all of it, 476 -> 175 us; one workgroup per CU, LDS 110 KB).
+// Rows of K, Q, V, T and P are staged in the order row(j) = 16 ((j >> 2) & 1) + 4 (j >> 3) + (j & 3) and the state's dk
+// rows alike within each 32, which makes accumulator tiles 0 and 1 of a lane group h hold tokens (dk) 8 h .. 8 h + 7 in
+// order: every operand is then one 16-byte LDS read in natural order, K^T and V^T two transposing reads. Y and O are taken transposed (the state as the A
+// operand), so a lane holds four neighbouring columns of a token and the outputs leave as 8-byte LDS writes.
+// row strides of 32 bytes past a multiple of 64: a fragment read (row lane % 16, 16 bytes at lane / 16) is then free
+// of bank conflicts (ds_read_b128 serves lanes 0-3, 12-15, 20-27 together, and so on: strides of 80 and 272 bytes
+// took two cycles for one, measured)
+constexpr int kRowK2 = kDk + 16;
+constexpr int kRowC = kC + 16;
+constexpr int kRowV = kCols + 8;
+constexpr int kRowO = kCols + 4;
+constexpr int kRoleThreads = 512;
+
+struct PStage {
+  uint16_t k[kC][kRowK2];
+  uint16_t q[kC][kRowK2];
+  uint16_t v[kC][kRowV];
+  uint16_t tm[2][kC][kRowC];      // T hi, lo
+  float vec[kVecN];
+};
+struct RoleLds {
+  PStage st[3];
+  uint16_t pm[2][2][kC][kRowC];   // P hi, lo of two chunks
+  uint16_t ob[2][kC][kRowO];      // outputs of two chunks
+};
+
+__device__ __forceinline__ int perm_row(int j) { return (j & ~31) + 16 * ((j >> 2) & 1) + 4 * ((j & 31) >> 3) + (j & 3); }
+// A barrier over LDS only: __syncthreads would also wait for the chunk loads in flight and for the output stores
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+// rows t0 .. of a [L, stride] bf16 matrix at `base` (its first row), at most one chunk of them: reads past the
+// sequence give zeros and writes past it are dropped
+__device__ __forceinline__ rsrc_t chunk_rsrc(const uint16_t* base, int64_t stride, int64_t t0, int64_t L) {
+  const int64_t rows = t0 < 0 || t0 >= L ? 0 : L - t0 < kC ? L - t0 : kC;
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(base + t0 * stride), (short)0, (int)(rows * stride * 2), 0x00020000);
+}
+__device__ __forceinline__ uint4 bload(rsrc_t r, int off) {
+  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+__global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs p) {
+  __shared__ __attribute__((aligned(16))) RoleLds sm;
+  const int nblk = p.dv / kCols;
+  // consecutive blocks of the (sequence, head, column block) order on one XCD: both column blocks and the value heads
+  // of a key head read the same K and Q
+  const unsigned nb = gridDim.x;
+  const int64_t bid = nb % 8 == 0 ? (int64_t)(blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int cb = (int)(bid % nblk);
+  const int h = (int)((bid / nblk) % p.n_v);
+  const int64_t s = bid / ((int64_t)nblk * p.n_v);
+  const int hk = h / (p.n_v / p.n_k);
+  const int tid = threadIdx.x % 256, lane = tid & 63, h4 = lane >> 4, lc = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), w = wv & 3;
+  const int64_t kd = (int64_t)p.n_k * kDk, ldv = (int64_t)p.n_v * p.dv;
+  const int64_t m0 = s * p.L;
+  const int n = (int)p.nchunk;
+  const float qscale = (float)0.08838834764831845;  // fp32(1 / sqrt(128)), the reference's query scale
+  const int otok = 8 * (lc >> 2) + (lc & 3);  // the token of row lc of tile 0 (of tile 1: + 4)
+
+  if (wv < 4) {
+    // ---- chain: element i of state tile 2 m + u is dk row 32 m + 8 h4 + 4 u + i of column `col`
+    const int col = cb * kCols + 16 * w + lc;
+    v4f S[8];
+    const int64_t sidx = p.seq_state ? (int64_t)p.seq_state[s] : s;
+    const bool has_init = p.init && sidx >= 0 && sidx < p.n_states;
+    const int64_t row0 = 8 * h4;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) S[r] = v4f{0, 0, 0, 0};
+    if (has_init) {
+      const float* src = p.init + ((sidx * p.n_v + h) * kDk + row0) * p.dv + col;
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[r][i] = src[(int64_t)(32 * (r >> 1) + 4 * (r & 1) + i) * p.dv];
+    }
+    bf16x8 th[2], tl[2], bv, kf[4][2], qf[4][2];
+    // K^T and V^T operands through transposing reads of the row-major stage: lane 4 e + c of a 16-lane group points at
+    // the 8-byte piece c of row e (token 8 h4 + e; the second read: + 4, 16 staged rows on) and lane j receives column
+    // j % 4 of piece j / 4 in the four rows
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    typedef __attribute__((address_space(3))) const char lds_char;
+    auto tr8 = [&](const void* at, int next) {
+      lds_char* src = (lds_char*)at;
+      const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)src);
+      const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(src + next));
+      return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    const int trow = 4 * h4 + (lc >> 2);
+    auto frags_kq = [&](const PStage& st) {
+      bv = tr8(&st.v[trow][16 * w + 4 * (lc & 3)], 16 * 2 * kRowV);  // 16 contiguous columns
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          kf[m][t] = lds8(&st.k[16 * t + lc][32 * m + 8 * h4]);
+          qf[m][t] = lds8(&st.q[16 * t + lc][32 * m + 8 * h4]);
+        }
+    };
+    auto frags_t = [&](const PStage& st) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        th[t] = lds8(&st.tm[0][16 * t + lc][8 * h4]);
+        tl[t] = lds8(&st.tm[1][16 * t + lc][8 * h4]);
+      }
+    };
+    lds_barrier();
+    frags_kq(sm.st[0]);
+    frags_t(sm.st[0]);
+    lds_barrier();
+    int cur = 0;
+    for (int c = 0; c < n; ++c) {
+      const PStage& st = sm.st[cur];
+      cur = cur == 2 ? 0 : cur + 1;
+      const PStage& sn = sm.st[cur];  // chunk c + 1, whole since the last barrier (past the end: stale, unused)
+      const float elast = st.vec[3 * kC];
+      const float4 e0 = *reinterpret_cast<const float4*>(&st.vec[kC + 8 * h4]);
+      const float4 e1 = *reinterpret_cast<const float4*>(&st.vec[kC + 8 * h4 + 4]);
+      const float4 c0 = *reinterpret_cast<const float4*>(&st.vec[2 * kC + 8 * h4]);
+      const float4 c1 = *reinterpret_cast<const float4*>(&st.vec[2 * kC + 8 * h4 + 4]);
+      const float eq[2] = {st.vec[kC + otok] * qscale, st.vec[kC + otok + 4] * qscale};
+      v4f X[2], Y[2], D[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        X[t] = v4f{0, 0, 0, 0};
+        Y[t] = v4f{0, 0, 0, 0};
+        D[t] = mfma16(th[t], bv, v4f{0, 0, 0, 0});  // U = T V
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) D[t] = mfma16(tl[t], bv, D[t]);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        bf16x8 sh, sl;
+        acc_to_b(S[2 * m], S[2 * m + 1], sh, sl);
+        X[0] = mfma16(kf[m][0], sh, X[0]);
+        X[1] = mfma16(kf[m][1], sh, X[1]);
+        Y[0] = mfma16(sh, qf[m][0], Y[0]);
+        Y[1] = mfma16(sh, qf[m][1], Y[1]);
+        X[0] = mfma16(kf[m][0], sl, X[0]);
+        X[1] = mfma16(kf[m][1], sl, X[1]);
+        Y[0] = mfma16(sl, qf[m][0], Y[0]);
+        Y[1] = mfma16(sl, qf[m][1], Y[1]);
+        S[2 * m] *= elast;
+        S[2 * m + 1] *= elast;
+      }
+      bf16x8 kt[8], ph[2], pl[2];
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        kt[r] = tr8(&st.k[trow][32 * (r >> 1) + 8 * (lc & 3) + 4 * (r & 1)], 16 * 2 * kRowK2);
+      // delta = U - T (diag(e^gamma) X)
+      bf16x8 xh, xl;
+      acc_to_b(v4f{-e0.x, -e0.y, -e0.z, -e0.w} * X[0], v4f{-e1.x, -e1.y, -e1.z, -e1.w} * X[1], xh, xl);
+      D[0] = mfma16(th[0], xh, D[0]);
+      D[1] = mfma16(th[1], xh, D[1]);
+      D[0] = mfma16(th[0], xl, D[0]);
+      D[1] = mfma16(th[1], xl, D[1]);
+      D[0] = mfma16(tl[0], xh, D[0]);
+      D[1] = mfma16(tl[1], xh, D[1]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        ph[t] = lds8(&sm.pm[c & 1][0][16 * t + lc][8 * h4]);
+        pl[t] = lds8(&sm.pm[c & 1][1][16 * t + lc][8 * h4]);
+      }
+      frags_kq(sn);
+      frags_t(sn);
+      // S = e^{gamma_C} S_0 + K^T diag(e^{gamma_C - gamma}) delta
+      bf16x8 eh, el, dh, dl;
+      acc_to_b(v4f{c0.x, c0.y, c0.z, c0.w} * D[0], v4f{c1.x, c1.y, c1.z, c1.w} * D[1], eh, el);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) S[r] = mfma16(kt[r], eh, S[r]);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) S[r] = mfma16(kt[r], el, S[r]);
+      // O^T = Y^T diag(e^gamma / sqrt(dk)) + delta^T P^T
+      acc_to_b(D[0], D[1], dh, dl);
+      v4f O[2] = {Y[0] * eq[0], Y[1] * eq[1]};
+#pragma unroll
+      for (int t = 0; t < 2; ++t) O[t] = mfma16(dh, ph[t], O[t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) O[t] = mfma16(dl, ph[t], O[t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) O[t] = mfma16(dh, pl[t], O[t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        *reinterpret_cast<uint2*>(&sm.ob[c & 1][16 * t + lc][16 * w + 4 * h4]) =
+            make_uint2(od_pack_bf16x2(O[t][0], O[t][1]), od_pack_bf16x2(O[t][2], O[t][3]));
+      lds_barrier();
+    }
+    if (p.final_state) {
+      float* dst = p.final_state + ((s * p.n_v + h) * kDk + row0) * p.dv + col;
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dst[(int64_t)(32 * (r >> 1) + 4 * (r & 1) + i) * p.dv] = S[r][i];
+    }
+  } else {
+    // ---- staging: rows of K, Q and V (16 lanes of 16 bytes, or 8, per row), T and the vectors through registers, two
+    // sets: a chunk is loaded two steps before it is written to LDS
+    const uint16_t* qk0 = p.qk + m0 * 2 * kd + (int64_t)hk * kDk;
+    const uint16_t* v0 = p.v + m0 * ldv + (int64_t)h * p.dv + cb * kCols;
+    uint16_t* o0 = p.o + m0 * ldv + (int64_t)h * p.dv + cb * kCols;
+    const uint4* ws0 = reinterpret_cast<const uint4*>(p.ws + (s * p.nchunk * p.n_v + h) * (int64_t)kTWs);
+    const int tj = ((tid >> 3) & 1) | ((tid >> 2) & 1) << 1 | ((tid >> 4) & 7) << 2, tq = tid & 3;  // row, part of T
+    const int rb = (int)(4 * kd), qo = (tid >> 4) * rb + 16 * (tid & 15), ko = qo + (int)(2 * kd);
+    const int vo = (tid >> 3) * (int)(2 * ldv) + 16 * (tid & 7);
+    // Every load is unconditional (chunks past the end: no rows, the last T block again), so that the compiler knows
+    // how many are in flight and each use waits for its own loads only
+    struct Pre {
+      uint4 k0, k1, q0, q1, v0, w0, vec;
+    };
+    auto gload = [&](int c, Pre& r) {
+      const rsrc_t rq = chunk_rsrc(qk0, 2 * kd, (int64_t)c * kC, p.L), rv = chunk_rsrc(v0, ldv, (int64_t)c * kC, p.L);
+      r.k0 = bload(rq, ko);
+      r.k1 = bload(rq, ko + 16 * rb);
+      r.q0 = bload(rq, qo);
+      r.q1 = bload(rq, qo + 16 * rb);
+      r.v0 = bload(rv, vo);
+      const uint4* blk = ws0 + (int64_t)(c < n ? c : n - 1) * p.n_v * (kTWs / 4);
+      r.w0 = blk[(tid >> 7) * (kMat / 8) + 4 * tj + tq];                       // T hi, lo: 256 pieces
+      r.vec = blk[2 * kMat / 8 + (tid < kVecN / 4 ? tid : kVecN / 4 - 1)];     // the vectors: 28 pieces
+    };
+    auto swrite = [&](PStage& st, const Pre& r) {
+      const int r0 = perm_row(tid >> 4);  // row 16 + (tid >> 4): 8 staged rows on
+      *reinterpret_cast<uint4*>(&st.k[r0][8 * (tid & 15)]) = r.k0;
+      *reinterpret_cast<uint4*>(&st.k[r0 + 8][8 * (tid & 15)]) = r.k1;
+      *reinterpret_cast<uint4*>(&st.q[r0][8 * (tid & 15)]) = r.q0;
+      *reinterpret_cast<uint4*>(&st.q[r0 + 8][8 * (tid & 15)]) = r.q1;
+      *reinterpret_cast<uint4*>(&st.v[perm_row(tid >> 3)][8 * (tid & 7)]) = r.v0;
+      *reinterpret_cast<uint4*>(&st.tm[tid >> 7][perm_row(tj)][8 * tq]) = r.w0;
+      if (tid < kVecN / 4) *reinterpret_cast<uint4*>(&st.vec[4 * tid]) = r.vec;
+    };
+    // P^T = K Q~^T o D^T, one 16 x 16 tile per wave: keys 8 h4 + 4 tk + r, query i
+    auto pmat = [&](const PStage& st, uint16_t (*pm)[kC][kRowC]) {
+      const int tk = w >> 1, ti = w & 1;
+      v4f a = {0, 0, 0, 0};
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        a = mfma16(lds8(&st.k[16 * tk + lc][32 * m + 8 * h4]), lds8(&st.q[16 * ti + lc][32 * m + 8 * h4]), a);
+      const int i = otok + 4 * ti, j0 = 8 * h4 + 4 * tk;
+      const float gi = st.vec[i];
+      const float4 gj = *reinterpret_cast<const float4*>(&st.vec[j0]);
+      const float gv[4] = {gj.x, gj.y, gj.z, gj.w};
+      float pv[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool seen = j0 + r <= i;
+        const float e = a[r] * qscale * __expf(seen ? gi - gv[r] : 0.0f);  // both selects: no branch
+        pv[r] = seen ? e : 0.0f;
+      }
+      uint32_t hi0, lo0, hi1, lo1;
+      split2(pv[0], pv[1], hi0, lo0);
+      split2(pv[2], pv[3], hi1, lo1);
+      *reinterpret_cast<uint2*>(&pm[0][16 * ti + lc][j0]) = make_uint2(hi0, hi1);
+      *reinterpret_cast<uint2*>(&pm[1][16 * ti + lc][j0]) = make_uint2(lo0, lo1);
+    };
+    auto store = [&](int c) {
+      const rsrc_t ro = chunk_rsrc(o0, ldv, (int64_t)c * kC, p.L);
+      typedef int v4i __attribute__((ext_vector_type(4)));
+      const uint2* src = reinterpret_cast<const uint2*>(&sm.ob[c & 1][perm_row(tid >> 3)][8 * (tid & 7)]);
+      const uint2 a = src[0], b = src[1];
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_uint4(a.x, a.y, b.x, b.y)), ro,
+                                             (tid >> 3) * (int)(2 * ldv) + 16 * (tid & 7), 0, 0);
+    };
+    Pre pa, pb;
+    gload(0, pa);
+    gload(1, pb);
+    swrite(sm.st[0], pa);
+    gload(2, pa);
+    swrite(sm.st[1], pb);
+    gload(3, pb);
+    lds_barrier();
+    pmat(sm.st[0], sm.pm[0]);
+    lds_barrier();
+    int nxt = 1;  // stage of chunk c + 1
+    // (past the last chunk the stages and P written here are not read)
+    auto step = [&](int c, Pre& r) {
+      const int two = nxt == 2 ? 0 : nxt + 1;
+      swrite(sm.st[two], r);
+      gload(c + 4, r);
+      store(c - 1);
+      pmat(sm.st[nxt], sm.pm[(c + 1) & 1]);
+      nxt = two;
+      lds_barrier();
+    };
+    for (int c = 0;; c += 2) {
+      step(c, pa);
+      if (c + 1 >= n) break;
+      step(c + 1, pb);
+      if (c + 2 >= n) break;
+    }
+    store(n - 1);
+  }
+}
+
 }  // namespace
 
 extern "C" int od_gdn_chunk_ws_size(int64_t S, int64_t L, int64_t n_v, int64_t* ws_floats) {
@@ -482,6 +789,12 @@ extern "C" int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, 
   TArgs tp{qk, g, beta, ws, L, nchunk, (int)n_k, (int)n_v};
   gdn_chunk_t_kernel<<<dim3((unsigned)tblocks), dim3(64), 0, (hipStream_t)stream>>>(tp);
   CArgs cp{qk, v, init, seq_state, ws, o, final_state, L, nchunk, n_states, (int)n_k, (int)n_v, (int)dv};
-  gdn_chunk_state_kernel<<<dim3((unsigned)cblocks), dim3(256), 0, (hipStream_t)stream>>>(cp);
+  // Two or more chunks: a role per wave (4 x 4096 tokens, 32 heads, both kernels: 508 -> 231 us; 1 x 8192: 887 -> 322;
+  // 2 chunks of 64 sequences: 115 -> 112). Its one workgroup per CU loses to three of the other where two chunks come
+  // with more work than about 16 workgroups per CU (2 chunks of 256 sequences: 385 -> 401).
+  if (nchunk > 2 || (nchunk == 2 && cblocks <= 4096))
+    gdn_chunk_roles_kernel<<<dim3((unsigned)cblocks), dim3(kRoleThreads), 0, (hipStream_t)stream>>>(cp);
+  else
+    gdn_chunk_state_kernel<<<dim3((unsigned)cblocks), dim3(256), 0, (hipStream_t)stream>>>(cp);
   return od_launch_status();
 }

@@ -179,6 +179,36 @@ def test_gdn_recurrence_matches_float64(gpu_lib, S, L, n_k, n_v, init, gmul, chu
     assert torch.allclose(fs.cpu(), st_r.float(), rtol=1e-5, atol=1e-5 * st_r.abs().max().item())
 
 
+@pytest.mark.parametrize("S,L,n_k,n_v,dv,gmul", [(2, 33, 2, 4, 128, 1), (3, 64, 1, 2, 64, 1), (1, 65, 2, 2, 128, -5e-4),
+                                                 (2, 128, 2, 6, 64, 1), (1, 161, 1, 8, 128, 1), (3, 193, 2, 4, 192, 1)])
+def test_gdn_chunk_chain_edges(gpu_lib, S, L, n_k, n_v, dv, gmul):
+    """The chunk chain at 2 to 7 chunks, whole and partial last ones, 1 to 3 column blocks per head, block counts that
+    are and are not multiples of 8, growing gates (gmul < 0), started from shared states: the bars of
+    test_gdn_recurrence_matches_float64. Those hold where the terms of an output are not much larger than the output:
+    every product keeps 16 bits, so a growth of e^G over the sequence leaves 2^-16 e^G of the state in an output. The
+    gates here sum to about -900 (2000 at the largest A), so gmul = -5e-4 keeps e^G under 3 (at -0.01 the state grows
+    by e^9 to e^20 and outputs that cancel to its 2^-16 miss the one-step bar)."""
+    from opendecider_amd import kernels
+    g = torch.Generator().manual_seed(S * 1000 + L + dv)
+    q, k, v, gg, beta = _rec_inputs(g, S, L, n_k, n_v, dv=dv)
+    gg = gg * gmul
+    st0 = torch.randn(2, n_v, 128, dv, generator=g) * 0.5
+    seq = torch.randint(0, 2, (S,), generator=g, dtype=torch.int32)
+    print(f"gdn chain S={S} L={L} n_k={n_k} n_v={n_v} dv={dv}", flush=True)
+    qk = torch.cat([q.reshape(S * L, -1), k.reshape(S * L, -1)], 1)
+    o, fs = kernels.gdn_recurrence(qk.to(DEV), v.reshape(S * L, -1).to(DEV), gg.to(DEV), beta.to(DEV), S, L, n_k, n_v,
+                                   128, dv, st0.to(DEV), seq.to(DEV), final=True)
+    rep = n_v // n_k
+    o_r, st_r = og.recurrence(q.repeat_interleave(rep, 1).reshape(S, L, n_v, 128),
+                              k.repeat_interleave(rep, 1).reshape(S, L, n_v, 128), v.reshape(S, L, n_v, dv),
+                              gg.reshape(S, L, n_v), beta.reshape(S, L, n_v), st0[seq.long()], torch.float64)
+    o_r = o_r.reshape(S * L, n_v * dv).float()
+    d = (o.cpu().float() - o_r).abs()
+    assert (d <= o_r.abs() * 2.0 ** -7 + 1e-6).all(), d.max().item()
+    assert (d.norm() / o_r.norm()).item() <= 2e-3
+    assert torch.allclose(fs.cpu(), st_r.float(), rtol=1e-5, atol=1e-5 * st_r.abs().max().item())
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 def test_gdn_recurrence_in_place_state_and_continuation(gpu_lib, chunked):
     """Running L1 tokens, then L2 more continuing the written state in place, equals one run over L1 + L2 tokens up
