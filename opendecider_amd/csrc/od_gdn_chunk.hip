@@ -219,6 +219,8 @@ struct CArgs {
   float* final_state;
   int64_t L, nchunk, n_states;
   int n_k, n_v, dv;
+  int64_t S;
+  int run;  // gdn_chunk_roles<true>: sequences per workgroup
 };
 
 constexpr int kRowK = kDk + 8;    // K, Q rows (272 bytes: conflict-free 8-byte reads per half-wave)
@@ -479,21 +481,22 @@ __global__ __launch_bounds__(256) void gdn_chunk_state_kernel(CArgs p) {
 // took two cycles for one, measured)
 constexpr int kRowK2 = kDk + 16;
 constexpr int kRowC = kC + 16;
-constexpr int kRowV = kCols + 8;
-constexpr int kRowO = kCols + 4;
-constexpr int kRoleThreads = 512;
+constexpr int kChain = 4, kRowChain = 8;  // chain waves of a workgroup, 16 columns each
+constexpr int kMaxRun = 64;               // sequences of a row workgroup (their state indices sit one per lane)
 
-struct PStage {
-  uint16_t k[kC][kRowK2];
-  uint16_t q[kC][kRowK2];
-  uint16_t v[kC][kRowV];
-  uint16_t tm[2][kC][kRowC];      // T hi, lo
-  float vec[kVecN];
-};
+template <int NC>
 struct RoleLds {
-  PStage st[3];
+  static constexpr int kV = 16 * NC + (NC == 8 ? 16 : 8);  // row strides of V (conflict-free transposing reads) and O
+  static constexpr int kO = 16 * NC + 4;
+  struct Stage {
+    uint16_t k[kC][kRowK2];
+    uint16_t q[kC][kRowK2];
+    uint16_t v[kC][kV];
+    uint16_t tm[2][kC][kRowC];    // T hi, lo
+    float vec[kVecN];
+  } st[3];
   uint16_t pm[2][2][kC][kRowC];   // P hi, lo of two chunks
-  uint16_t ob[2][kC][kRowO];      // outputs of two chunks
+  uint16_t ob[2][kC][kO];         // outputs of two chunks
 };
 
 __device__ __forceinline__ int perm_row(int j) { return (j & ~31) + 16 * ((j >> 2) & 1) + 4 * ((j & 31) >> 3) + (j & 3); }
@@ -511,40 +514,59 @@ __device__ __forceinline__ uint4 bload(rsrc_t r, int off) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
 
-__global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs p) {
-  __shared__ __attribute__((aligned(16))) RoleLds sm;
-  const int nblk = p.dv / kCols;
-  // consecutive blocks of the (sequence, head, column block) order on one XCD: both column blocks and the value heads
-  // of a key head read the same K and Q
+// ROWS false: step c is chunk c of one sequence. ROWS true: one-chunk sequences that keep no final state (option rows),
+// step c is sequence s0 + c of a run that shares the head; S_0 is read and split only where the state index changes,
+// there is no update, and eight chain waves cover 128 columns.
+template <bool ROWS>
+__global__ __launch_bounds__(64 * (ROWS ? kRowChain + 4 : kChain + 4), ROWS ? 3 : 2) void gdn_chunk_roles_kernel(CArgs p) {
+  constexpr int NC = ROWS ? kRowChain : kChain, COLS = 16 * NC;
+  typedef RoleLds<NC> Lds;
+  typedef typename Lds::Stage Stage;
+  __shared__ __attribute__((aligned(16))) Lds sm;
+  const int nblk = p.dv / COLS;
+  // consecutive blocks of the (sequence or run, head, column block) order on one XCD: both column blocks and the value
+  // heads of a key head read the same K and Q
   const unsigned nb = gridDim.x;
   const int64_t bid = nb % 8 == 0 ? (int64_t)(blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8 : blockIdx.x;
   const int cb = (int)(bid % nblk);
   const int h = (int)((bid / nblk) % p.n_v);
-  const int64_t s = bid / ((int64_t)nblk * p.n_v);
+  const int64_t s = bid / ((int64_t)nblk * p.n_v) * (ROWS ? p.run : 1);  // the (first) sequence
   const int hk = h / (p.n_v / p.n_k);
-  const int tid = threadIdx.x % 256, lane = tid & 63, h4 = lane >> 4, lc = lane & 15;
-  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), w = wv & 3;
+  const int lane = threadIdx.x & 63, h4 = lane >> 4, lc = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int64_t kd = (int64_t)p.n_k * kDk, ldv = (int64_t)p.n_v * p.dv;
+  const int n = ROWS ? (int)min((int64_t)p.run, p.S - s) : (int)p.nchunk;
   const int64_t m0 = s * p.L;
-  const int n = (int)p.nchunk;
   const float qscale = (float)0.08838834764831845;  // fp32(1 / sqrt(128)), the reference's query scale
   const int otok = 8 * (lc >> 2) + (lc & 3);  // the token of row lc of tile 0 (of tile 1: + 4)
 
-  if (wv < 4) {
+  if (w < NC) {
     // ---- chain: element i of state tile 2 m + u is dk row 32 m + 8 h4 + 4 u + i of column `col`
-    const int col = cb * kCols + 16 * w + lc;
+    const int col = cb * COLS + 16 * w + lc;
     v4f S[8];
-    const int64_t sidx = p.seq_state ? (int64_t)p.seq_state[s] : s;
-    const bool has_init = p.init && sidx >= 0 && sidx < p.n_states;
     const int64_t row0 = 8 * h4;
+    auto load_state = [&](int64_t sidx) {
 #pragma unroll
-    for (int r = 0; r < 8; ++r) S[r] = v4f{0, 0, 0, 0};
-    if (has_init) {
-      const float* src = p.init + ((sidx * p.n_v + h) * kDk + row0) * p.dv + col;
+      for (int r = 0; r < 8; ++r) S[r] = v4f{0, 0, 0, 0};
+      if (p.init && sidx >= 0 && sidx < p.n_states) {
+        const float* src = p.init + ((sidx * p.n_v + h) * kDk + row0) * p.dv + col;
 #pragma unroll
-      for (int r = 0; r < 8; ++r)
+        for (int r = 0; r < 8; ++r)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[r][i] = src[(int64_t)(32 * (r >> 1) + 4 * (r & 1) + i) * p.dv];
+          for (int i = 0; i < 4; ++i) S[r][i] = src[(int64_t)(32 * (r >> 1) + 4 * (r & 1) + i) * p.dv];
+      }
+    };
+    bf16x8 sh[4], sl[4];
+    int states = 0, held = -1;  // ROWS: lane l holds the state index of sequence s + l (-1: none); the index in sh, sl
+    if constexpr (ROWS) {
+      if (lane < n) {
+        const int64_t x = p.seq_state ? (int64_t)p.seq_state[s + lane] : s + lane;
+        states = p.init && x >= 0 && x < p.n_states ? (int)x : -1;
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m) sh[m] = sl[m] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+    } else {
+      load_state(p.seq_state ? (int64_t)p.seq_state[s] : s);
     }
     bf16x8 th[2], tl[2], bv, kf[4][2], qf[4][2];
     // K^T and V^T operands through transposing reads of the row-major stage: lane 4 e + c of a 16-lane group points at
@@ -560,8 +582,8 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
       return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
     };
     const int trow = 4 * h4 + (lc >> 2);
-    auto frags_kq = [&](const PStage& st) {
-      bv = tr8(&st.v[trow][16 * w + 4 * (lc & 3)], 16 * 2 * kRowV);  // 16 contiguous columns
+    auto frags_kq = [&](const Stage& st) {
+      bv = tr8(&st.v[trow][16 * w + 4 * (lc & 3)], 16 * 2 * Lds::kV);  // 16 contiguous columns
 #pragma unroll
       for (int m = 0; m < 4; ++m)
 #pragma unroll
@@ -570,7 +592,7 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
           qf[m][t] = lds8(&st.q[16 * t + lc][32 * m + 8 * h4]);
         }
     };
-    auto frags_t = [&](const PStage& st) {
+    auto frags_t = [&](const Stage& st) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         th[t] = lds8(&st.tm[0][16 * t + lc][8 * h4]);
@@ -578,14 +600,27 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
       }
     };
     lds_barrier();
-    frags_kq(sm.st[0]);
-    frags_t(sm.st[0]);
+    if constexpr (!ROWS) {
+      frags_kq(sm.st[0]);
+      frags_t(sm.st[0]);
+    }
     lds_barrier();
     int cur = 0;
     for (int c = 0; c < n; ++c) {
-      const PStage& st = sm.st[cur];
+      const Stage& st = sm.st[cur];
       cur = cur == 2 ? 0 : cur + 1;
-      const PStage& sn = sm.st[cur];  // chunk c + 1, whole since the last barrier (past the end: stale, unused)
+      const Stage& sn = sm.st[cur];  // chunk c + 1, whole since the last barrier (past the end: stale, unused)
+      if constexpr (ROWS) {  // two chain waves per SIMD hide each other's reads: no operands held across a barrier
+        frags_kq(st);
+        frags_t(st);
+        const int want = __builtin_amdgcn_readlane(states, c);
+        if (want != held) {
+          held = want;
+          load_state(want);
+#pragma unroll
+          for (int m = 0; m < 4; ++m) acc_to_b(S[2 * m], S[2 * m + 1], sh[m], sl[m]);
+        }
+      }
       const float elast = st.vec[3 * kC];
       const float4 e0 = *reinterpret_cast<const float4*>(&st.vec[kC + 8 * h4]);
       const float4 e1 = *reinterpret_cast<const float4*>(&st.vec[kC + 8 * h4 + 4]);
@@ -603,22 +638,29 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
       for (int t = 0; t < 2; ++t) D[t] = mfma16(tl[t], bv, D[t]);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        bf16x8 sh, sl;
-        acc_to_b(S[2 * m], S[2 * m + 1], sh, sl);
-        X[0] = mfma16(kf[m][0], sh, X[0]);
-        X[1] = mfma16(kf[m][1], sh, X[1]);
-        Y[0] = mfma16(sh, qf[m][0], Y[0]);
-        Y[1] = mfma16(sh, qf[m][1], Y[1]);
-        X[0] = mfma16(kf[m][0], sl, X[0]);
-        X[1] = mfma16(kf[m][1], sl, X[1]);
-        Y[0] = mfma16(sl, qf[m][0], Y[0]);
-        Y[1] = mfma16(sl, qf[m][1], Y[1]);
-        S[2 * m] *= elast;
-        S[2 * m + 1] *= elast;
+        bf16x8 ah, al;
+        if constexpr (ROWS) {
+          ah = sh[m];
+          al = sl[m];
+        } else {
+          acc_to_b(S[2 * m], S[2 * m + 1], ah, al);
+        }
+        X[0] = mfma16(kf[m][0], ah, X[0]);
+        X[1] = mfma16(kf[m][1], ah, X[1]);
+        Y[0] = mfma16(ah, qf[m][0], Y[0]);
+        Y[1] = mfma16(ah, qf[m][1], Y[1]);
+        X[0] = mfma16(kf[m][0], al, X[0]);
+        X[1] = mfma16(kf[m][1], al, X[1]);
+        Y[0] = mfma16(al, qf[m][0], Y[0]);
+        Y[1] = mfma16(al, qf[m][1], Y[1]);
+        if constexpr (!ROWS) {
+          S[2 * m] *= elast;
+          S[2 * m + 1] *= elast;
+        }
       }
       bf16x8 kt[8], ph[2], pl[2];
 #pragma unroll
-      for (int r = 0; r < 8; ++r)
+      for (int r = 0; r < (ROWS ? 0 : 8); ++r)
         kt[r] = tr8(&st.k[trow][32 * (r >> 1) + 8 * (lc & 3) + 4 * (r & 1)], 16 * 2 * kRowK2);
       // delta = U - T (diag(e^gamma) X)
       bf16x8 xh, xl;
@@ -634,15 +676,17 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
         ph[t] = lds8(&sm.pm[c & 1][0][16 * t + lc][8 * h4]);
         pl[t] = lds8(&sm.pm[c & 1][1][16 * t + lc][8 * h4]);
       }
-      frags_kq(sn);
-      frags_t(sn);
-      // S = e^{gamma_C} S_0 + K^T diag(e^{gamma_C - gamma}) delta
       bf16x8 eh, el, dh, dl;
-      acc_to_b(v4f{c0.x, c0.y, c0.z, c0.w} * D[0], v4f{c1.x, c1.y, c1.z, c1.w} * D[1], eh, el);
+      if constexpr (!ROWS) {
+        frags_kq(sn);
+        frags_t(sn);
+        // S = e^{gamma_C} S_0 + K^T diag(e^{gamma_C - gamma}) delta
+        acc_to_b(v4f{c0.x, c0.y, c0.z, c0.w} * D[0], v4f{c1.x, c1.y, c1.z, c1.w} * D[1], eh, el);
 #pragma unroll
-      for (int r = 0; r < 8; ++r) S[r] = mfma16(kt[r], eh, S[r]);
+        for (int r = 0; r < 8; ++r) S[r] = mfma16(kt[r], eh, S[r]);
 #pragma unroll
-      for (int r = 0; r < 8; ++r) S[r] = mfma16(kt[r], el, S[r]);
+        for (int r = 0; r < 8; ++r) S[r] = mfma16(kt[r], el, S[r]);
+      }
       // O^T = Y^T diag(e^gamma / sqrt(dk)) + delta^T P^T
       acc_to_b(D[0], D[1], dh, dl);
       v4f O[2] = {Y[0] * eq[0], Y[1] * eq[1]};
@@ -658,7 +702,7 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
             make_uint2(od_pack_bf16x2(O[t][0], O[t][1]), od_pack_bf16x2(O[t][2], O[t][3]));
       lds_barrier();
     }
-    if (p.final_state) {
+    if (!ROWS && p.final_state) {
       float* dst = p.final_state + ((s * p.n_v + h) * kDk + row0) * p.dv + col;
 #pragma unroll
       for (int r = 0; r < 8; ++r)
@@ -669,41 +713,50 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
     // ---- staging: rows of K, Q and V (16 lanes of 16 bytes, or 8, per row), T and the vectors through registers, two
     // sets: a chunk is loaded two steps before it is written to LDS
     const uint16_t* qk0 = p.qk + m0 * 2 * kd + (int64_t)hk * kDk;
-    const uint16_t* v0 = p.v + m0 * ldv + (int64_t)h * p.dv + cb * kCols;
-    uint16_t* o0 = p.o + m0 * ldv + (int64_t)h * p.dv + cb * kCols;
-    const uint4* ws0 = reinterpret_cast<const uint4*>(p.ws + (s * p.nchunk * p.n_v + h) * (int64_t)kTWs);
+    const int tid = threadIdx.x - 64 * NC, ws = w - NC;  // thread and wave of the four
+    const uint16_t* v0 = p.v + m0 * ldv + (int64_t)h * p.dv + cb * COLS;
+    uint16_t* o0 = p.o + m0 * ldv + (int64_t)h * p.dv + cb * COLS;
+    const uint4* tw0 = reinterpret_cast<const uint4*>(p.ws + (s * p.nchunk * p.n_v + h) * (int64_t)kTWs);
     const int tj = ((tid >> 3) & 1) | ((tid >> 2) & 1) << 1 | ((tid >> 4) & 7) << 2, tq = tid & 3;  // row, part of T
     const int rb = (int)(4 * kd), qo = (tid >> 4) * rb + 16 * (tid & 15), ko = qo + (int)(2 * kd);
-    const int vo = (tid >> 3) * (int)(2 * ldv) + 16 * (tid & 7);
+    constexpr int kParts = COLS / 8, kVRows = 256 / kParts;  // 16-byte parts of a V or O row, rows per pass of 256 threads
+    const int vr = tid / kParts, vp = tid % kParts, vo = vr * (int)(2 * ldv) + 16 * vp;
+    // step c: chunk c of the sequence, or the one chunk of sequence s + c
+    auto rows_of = [&](const uint16_t* base, int64_t stride, int c) {
+      if constexpr (ROWS) return chunk_rsrc(base + (int64_t)c * p.L * stride, stride, c >= 0 && c < n ? 0 : -1, p.L);
+      return chunk_rsrc(base, stride, (int64_t)c * kC, p.L);
+    };
     // Every load is unconditional (chunks past the end: no rows, the last T block again), so that the compiler knows
     // how many are in flight and each use waits for its own loads only
     struct Pre {
-      uint4 k0, k1, q0, q1, v0, w0, vec;
+      uint4 k0, k1, q0, q1, v0, v1, w0, vec;
     };
     auto gload = [&](int c, Pre& r) {
-      const rsrc_t rq = chunk_rsrc(qk0, 2 * kd, (int64_t)c * kC, p.L), rv = chunk_rsrc(v0, ldv, (int64_t)c * kC, p.L);
+      const rsrc_t rq = rows_of(qk0, 2 * kd, c), rv = rows_of(v0, ldv, c);
       r.k0 = bload(rq, ko);
       r.k1 = bload(rq, ko + 16 * rb);
       r.q0 = bload(rq, qo);
       r.q1 = bload(rq, qo + 16 * rb);
       r.v0 = bload(rv, vo);
-      const uint4* blk = ws0 + (int64_t)(c < n ? c : n - 1) * p.n_v * (kTWs / 4);
+      r.v1 = ROWS ? bload(rv, vo + kVRows * (int)(2 * ldv)) : r.v0;
+      const uint4* blk = tw0 + (int64_t)(c < n ? c : n - 1) * p.n_v * (kTWs / 4);
       r.w0 = blk[(tid >> 7) * (kMat / 8) + 4 * tj + tq];                       // T hi, lo: 256 pieces
       r.vec = blk[2 * kMat / 8 + (tid < kVecN / 4 ? tid : kVecN / 4 - 1)];     // the vectors: 28 pieces
     };
-    auto swrite = [&](PStage& st, const Pre& r) {
+    auto swrite = [&](Stage& st, const Pre& r) {
       const int r0 = perm_row(tid >> 4);  // row 16 + (tid >> 4): 8 staged rows on
       *reinterpret_cast<uint4*>(&st.k[r0][8 * (tid & 15)]) = r.k0;
       *reinterpret_cast<uint4*>(&st.k[r0 + 8][8 * (tid & 15)]) = r.k1;
       *reinterpret_cast<uint4*>(&st.q[r0][8 * (tid & 15)]) = r.q0;
       *reinterpret_cast<uint4*>(&st.q[r0 + 8][8 * (tid & 15)]) = r.q1;
-      *reinterpret_cast<uint4*>(&st.v[perm_row(tid >> 3)][8 * (tid & 7)]) = r.v0;
+      *reinterpret_cast<uint4*>(&st.v[perm_row(vr)][8 * vp]) = r.v0;
+      if constexpr (ROWS) *reinterpret_cast<uint4*>(&st.v[perm_row(vr + kVRows)][8 * vp]) = r.v1;
       *reinterpret_cast<uint4*>(&st.tm[tid >> 7][perm_row(tj)][8 * tq]) = r.w0;
       if (tid < kVecN / 4) *reinterpret_cast<uint4*>(&st.vec[4 * tid]) = r.vec;
     };
     // P^T = K Q~^T o D^T, one 16 x 16 tile per wave: keys 8 h4 + 4 tk + r, query i
-    auto pmat = [&](const PStage& st, uint16_t (*pm)[kC][kRowC]) {
-      const int tk = w >> 1, ti = w & 1;
+    auto pmat = [&](const Stage& st, uint16_t (*pm)[kC][kRowC]) {
+      const int tk = ws >> 1, ti = ws & 1;
       v4f a = {0, 0, 0, 0};
 #pragma unroll
       for (int m = 0; m < 4; ++m)
@@ -726,12 +779,15 @@ __global__ __launch_bounds__(kRoleThreads, 2) void gdn_chunk_roles_kernel(CArgs 
       *reinterpret_cast<uint2*>(&pm[1][16 * ti + lc][j0]) = make_uint2(lo0, lo1);
     };
     auto store = [&](int c) {
-      const rsrc_t ro = chunk_rsrc(o0, ldv, (int64_t)c * kC, p.L);
+      const rsrc_t ro = rows_of(o0, ldv, c);
       typedef int v4i __attribute__((ext_vector_type(4)));
-      const uint2* src = reinterpret_cast<const uint2*>(&sm.ob[c & 1][perm_row(tid >> 3)][8 * (tid & 7)]);
-      const uint2 a = src[0], b = src[1];
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_uint4(a.x, a.y, b.x, b.y)), ro,
-                                             (tid >> 3) * (int)(2 * ldv) + 16 * (tid & 7), 0, 0);
+#pragma unroll
+      for (int r = 0; r < kC; r += kVRows) {
+        const uint2* src = reinterpret_cast<const uint2*>(&sm.ob[c & 1][perm_row(vr + r)][8 * vp]);
+        const uint2 a = src[0], b = src[1];
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, make_uint4(a.x, a.y, b.x, b.y)), ro,
+                                               vo + r * (int)(2 * ldv), 0, 0);
+      }
     };
     Pre pa, pb;
     gload(0, pa);
@@ -788,12 +844,20 @@ extern "C" int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, 
   if (tblocks > 0x7fffffffll || cblocks > 0x7fffffffll || S * L > 0x7fffffffll) return OD_ERR_SHAPE;
   TArgs tp{qk, g, beta, ws, L, nchunk, (int)n_k, (int)n_v};
   gdn_chunk_t_kernel<<<dim3((unsigned)tblocks), dim3(64), 0, (hipStream_t)stream>>>(tp);
-  CArgs cp{qk, v, init, seq_state, ws, o, final_state, L, nchunk, n_states, (int)n_k, (int)n_v, (int)dv};
+  CArgs cp{qk, v, init, seq_state, ws, o, final_state, L, nchunk, n_states, (int)n_k, (int)n_v, (int)dv, S, 1};
+  // One chunk and no state kept (option rows): runs of sequences that share S_0 in registers, a workgroup per CU.
+  if (nchunk == 1 && !final_state && dv % (16 * kRowChain) == 0) {
+    const int64_t heads = n_v * (dv / (16 * kRowChain));
+    cp.run = (int)min((int64_t)kMaxRun, max((int64_t)1, S * heads / 256));
+    const int64_t blocks = (S + cp.run - 1) / cp.run * heads;
+    gdn_chunk_roles_kernel<true><<<dim3((unsigned)blocks), dim3(64 * (kRowChain + 4)), 0, (hipStream_t)stream>>>(cp);
+    return od_launch_status();
+  }
   // Two or more chunks: a role per wave (4 x 4096 tokens, 32 heads, both kernels: 508 -> 231 us; 1 x 8192: 887 -> 322;
   // 2 chunks of 64 sequences: 115 -> 112). Its one workgroup per CU loses to three of the other where two chunks come
   // with more work than about 16 workgroups per CU (2 chunks of 256 sequences: 385 -> 401).
   if (nchunk > 2 || (nchunk == 2 && cblocks <= 4096))
-    gdn_chunk_roles_kernel<<<dim3((unsigned)cblocks), dim3(kRoleThreads), 0, (hipStream_t)stream>>>(cp);
+    gdn_chunk_roles_kernel<false><<<dim3((unsigned)cblocks), dim3(64 * (kChain + 4)), 0, (hipStream_t)stream>>>(cp);
   else
     gdn_chunk_state_kernel<<<dim3((unsigned)cblocks), dim3(256), 0, (hipStream_t)stream>>>(cp);
   return od_launch_status();

@@ -209,6 +209,37 @@ def test_gdn_chunk_chain_edges(gpu_lib, S, L, n_k, n_v, dv, gmul):
     assert torch.allclose(fs.cpu(), st_r.float(), rtol=1e-5, atol=1e-5 * st_r.abs().max().item())
 
 
+@pytest.mark.parametrize("S,L,n_k,n_v,dv,states", [(1, 1, 2, 4, 128, 1), (3, 32, 1, 2, 128, 0), (200, 5, 2, 4, 128, 3),
+                                                   (130, 31, 1, 8, 128, 2), (70, 9, 2, 4, 256, 3), (5, 24, 2, 4, 64, 2)])
+def test_gdn_one_chunk_rows(gpu_lib, S, L, n_k, n_v, dv, states):
+    """Sequences of at most 32 tokens that keep no final state (option rows): runs of one and several sequences per
+    workgroup, a last run that is shorter, states in any order with one index outside the states (zeros), no states at
+    all, two column blocks, and the other kernel's dv = 64: the bars of test_gdn_recurrence_matches_float64."""
+    from opendecider_amd import kernels
+    g = torch.Generator().manual_seed(S * 1000 + L + dv)
+    q, k, v, gg, beta = _rec_inputs(g, S, L, n_k, n_v, dv=dv)
+    st0 = torch.randn(states, n_v, 128, dv, generator=g) * 0.5 if states else None
+    seq = torch.randint(0, states, (S,), generator=g, dtype=torch.int32) if states else None
+    if states > 1:
+        seq[S // 2] = states
+    print(f"gdn rows S={S} L={L} n_v={n_v} dv={dv} states={states}", flush=True)
+    qk = torch.cat([q.reshape(S * L, -1), k.reshape(S * L, -1)], 1)
+    o, fs = kernels.gdn_recurrence(qk.to(DEV), v.reshape(S * L, -1).to(DEV), gg.to(DEV), beta.to(DEV), S, L, n_k, n_v,
+                                   128, dv, None if st0 is None else st0.to(DEV), None if seq is None else seq.to(DEV))
+    assert fs is None
+    rep = n_v // n_k
+    init = None
+    if states:
+        init = torch.cat([st0, torch.zeros(1, n_v, 128, dv)])[seq.long()]
+    o_r, _ = og.recurrence(q.repeat_interleave(rep, 1).reshape(S, L, n_v, 128),
+                           k.repeat_interleave(rep, 1).reshape(S, L, n_v, 128), v.reshape(S, L, n_v, dv),
+                           gg.reshape(S, L, n_v), beta.reshape(S, L, n_v), init, torch.float64)
+    o_r = o_r.reshape(S * L, n_v * dv).float()
+    d = (o.cpu().float() - o_r).abs()
+    assert (d <= o_r.abs() * 2.0 ** -7 + 1e-6).all(), d.max().item()
+    assert (d.norm() / o_r.norm()).item() <= 2e-3
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 def test_gdn_recurrence_in_place_state_and_continuation(gpu_lib, chunked):
     """Running L1 tokens, then L2 more continuing the written state in place, equals one run over L1 + L2 tokens up
