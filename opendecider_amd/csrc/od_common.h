@@ -75,6 +75,15 @@ __device__ __forceinline__ float od_silu_bf16(float g) {
   return od_bf16_to_f32(od_f32_to_bf16(s));
 }
 
+// A table of bf16(silu(g)) (od_silu_bf16) for 2^-8 <= |g| < 16: bf16 patterns kSiluLo .. kSiluHi - 1 of each sign,
+// positive ones first (2 x 1536 entries, 6 KB); entry i of it.
+constexpr uint32_t kSiluLo = 0x3b80u, kSiluHi = 0x4180u, kSiluHalf = kSiluHi - kSiluLo;
+__device__ __forceinline__ uint16_t od_silu_table_entry(int i) {
+  const uint32_t h = (uint32_t)i >= kSiluHalf;
+  const uint32_t bits = (h << 15) | (kSiluLo + (uint32_t)i - h * kSiluHalf);
+  return od_f32_to_bf16(od_silu_bf16(__uint_as_float(bits << 16)));
+}
+
 // bf16(RN32(sigmoid(g))), sigmoid(g) = 1 / (1 + exp(-g)), for the output gate (torch.sigmoid on a bf16 tensor
 // computes in fp32 and rounds to bf16): the same exp(-g) as od_silu_bf16, then the sum and a reciprocal, within
 // 10 fp32 ulps; values within 16 ulps of a bf16 midpoint, and |g| >= 16, are recomputed in float64.

@@ -96,121 +96,217 @@ __device__ __forceinline__ float silu_bf16(float g) {
   return od_bf16_to_f32(od_f32_to_bf16(s));
 }
 
-// One workgroup per (tile of kTok consecutive tokens of one sequence, block of 8192 channels); thread i handles
-// channels 16 i .. 16 i + 15 of the block (a q / k head is dk / 16 consecutive threads, all in one wave) and slides
-// the conv window (the previous 3 inputs of its channels) along the tile in registers, so each input row is read
-// once per tile instead of four times.
-constexpr int kTok = 8;
-constexpr int kPrepThreads = 512;
+// One workgroup per (tile of kTok consecutive tokens of one sequence, block of kPrepThreads * NCH channels); thread i
+// handles channels NCH i .. + NCH - 1 of the block (a q / k head is dk / NCH consecutive threads, all in one wave) and
+// slides the conv window (the previous 3 inputs of its channels) along the tile in registers, four buffers in turn.
+//
+// The bytes are those of the float64 evaluation (conv sums and squares exact, rounded once); the pass is bound by
+// vector instructions and the latency behind them (4 x 4096 tokens: 62M wave instructions, 129M with float64 squares,
+// SiLUs by exp2 and a conversion per tap; 235 -> 168 us under the profiler, 542 MB at 5 TB/s would take 108; three
+// 4-wave workgroups per CU, 168 VGPRs: two waves per SIMD took 207), so they are few:
+//   conv    four float64 fma per channel on taps and a window kept in float64 (one conversion per input; an fp32 chain
+//           with an error bound fails it on 0.3% of channels, the ties of sums of 16-bit products)
+//   silu    of a bf16 value: a 6 KB LDS table of it for 2^-8 <= |g| < 16 and the exponent-decrement of g below (as the
+//           SwiGLU GEMM epilogue has it), in packed 16-bit steps over two channels; lanes with another g call the function
+//   l2norm  fp32 sum S of positive terms, off by at most 11 2^-24 S: bf16(S (1 - 2^-20)) == bf16(S (1 + 2^-20)) proves
+//           its rounding; rsq within 1 ulp, so its bf16 is right unless the low half lies within 4 ulps of the midpoint;
+//           else (1 wave in 200) float64
+constexpr int kTok = 16;
+constexpr int kPrepThreads = 256;
 
-__global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(PrepArgs p) {
+__device__ __forceinline__ float group_sum(float v, int G) {
+  if (G == 16) {
+    v = od_dpp_sum_step<0xB1, 0xf>(v);
+    v = od_dpp_sum_step<0x4E, 0xf>(v);
+    v = od_dpp_sum_step<0x124, 0xf>(v);
+    return od_dpp_sum_step<0x128, 0xf>(v);
+  }
+  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, OD_WAVE);
+  return v;
+}
+
+template <int NCH>
+__global__ __launch_bounds__(kPrepThreads, NCH == 8 ? 3 : 1) void gdn_prep_kernel(PrepArgs p) {
+  constexpr int NW = NCH / 2;  // words of bf16 pairs
+  __shared__ uint16_t stab[2 * kSiluHalf];
+  for (int i = threadIdx.x; i < (int)(2 * kSiluHalf); i += blockDim.x) stab[i] = od_silu_table_entry(i);
+  __syncthreads();
   const int64_t ntile = (p.L + kTok - 1) / kTok;
   const int64_t s = blockIdx.x / ntile, t0 = (blockIdx.x % ntile) * kTok;
   const int64_t m_s = s * p.L;  // first token of the sequence
   const int tid = threadIdx.x;
-  const int c0 = ((int)blockIdx.y * kPrepThreads + tid) * kChan;
+  const int c0 = ((int)blockIdx.y * (int)blockDim.x + tid) * NCH;
   const bool on = c0 < p.C;
   const int64_t st = p.seq_state ? (int64_t)p.seq_state[s] : s;
   const bool st_ok = p.conv_in != nullptr && st >= 0 && st < p.n_states;
   const int kd = p.n_k * p.dk;
-  const int G = p.dk / kChan;  // lanes per head (a power of two <= 64)
+  const int G = p.dk / NCH;  // lanes per head (a power of two <= 64)
   const int tn = (int)min((int64_t)kTok, p.L - t0);
   // real tokens of the sequence (clamped into [0, L]); tokens at or past it are right pads
   const int64_t len = p.seq_len ? min(max((int64_t)p.seq_len[s], (int64_t)0), p.L) : p.L;
 
-  // row r of full = [state (3 rows) ; the sequence's tokens]: full[r] = state row r (r < 3) or token r - 3, as 8
-  // words of bf16 pairs (the window and the next row stay in this raw form: half the registers of fp32)
-  auto load_full = [&](int64_t r, uint32_t (&x)[kChan / 2]) {
+  // row r of full = [state (3 rows) ; the sequence's tokens]: full[r] = state row r (r < 3) or token r - 3, as words of
+  // bf16 pairs
+  auto load_full = [&](int64_t r, uint32_t (&x)[NW]) {
     const uint16_t* src = nullptr;
     if (r >= kConvTaps - 1) src = p.proj + (m_s + r - (kConvTaps - 1)) * p.ldp + c0;
     else if (st_ok) src = p.conv_in + (st * (kConvTaps - 1) + r) * p.C + c0;
-    if (src) {
-      const uint4 lo = *reinterpret_cast<const uint4*>(src), hi = *reinterpret_cast<const uint4*>(src + 8);
-      x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w; x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
-    } else {
 #pragma unroll
-      for (int i = 0; i < kChan / 2; ++i) x[i] = 0u;
+    for (int i = 0; i < NW; i += 4) {
+      const uint4 v = src ? *reinterpret_cast<const uint4*>(src + 2 * i) : make_uint4(0, 0, 0, 0);
+      x[i] = v.x; x[i + 1] = v.y; x[i + 2] = v.z; x[i + 3] = v.w;
     }
   };
-  auto store_raw = [&](uint16_t* dst, const uint32_t (&x)[kChan / 2]) {
-    *reinterpret_cast<uint4*>(dst) = make_uint4(x[0], x[1], x[2], x[3]);
-    *reinterpret_cast<uint4*>(dst + 8) = make_uint4(x[4], x[5], x[6], x[7]);
+  auto unpack = [](const uint32_t (&x)[NW], float (&f)[NCH]) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      f[2 * i] = __uint_as_float(x[i] << 16);
+      f[2 * i + 1] = __uint_as_float(x[i] & 0xffff0000u);
+    }
   };
-  // channel i of a raw row, as fp32
-  auto chan = [](const uint32_t (&x)[kChan / 2], int i) {
-    return __uint_as_float((i & 1) ? (x[i >> 1] & 0xffff0000u) : (x[i >> 1] << 16));
+  auto widen = [](const uint32_t (&x)[NW], double (&f)[NCH]) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      f[2 * i] = (double)__uint_as_float(x[i] << 16);
+      f[2 * i + 1] = (double)__uint_as_float(x[i] & 0xffff0000u);
+    }
   };
-  uint32_t wr[kChan * kConvTaps / 2];  // the conv taps of this thread's channels, bf16 pairs (channel i: 2 words)
-  uint32_t win[kConvTaps - 1][kChan / 2];  // full rows t0 .. t0 + 2 (the inputs before token t0)
+  double w[kConvTaps][NCH];  // the taps of this thread's channels
+  double wa[NCH], wb[NCH], wc[NCH], wd[NCH];  // the window (three rows before a token) and the token's row, in turn
+  uint32_t xr[2][NW];  // the rows of this token and the next, raw: loads go out two tokens ahead
+#pragma unroll
+  for (int i = 0; i < NW; ++i) xr[0][i] = xr[1][i] = 0u;
   if (on) {
 #pragma unroll
-    for (int i = 0; i < kChan * kConvTaps / 8; ++i)
-      *reinterpret_cast<uint4*>(&wr[4 * i]) = *reinterpret_cast<const uint4*>(p.conv_w + (int64_t)c0 * kConvTaps + 8 * i);
+    for (int i = 0; i < NCH; i += 2) {  // two channels of four taps: 16 bytes
+      const uint4 v = *reinterpret_cast<const uint4*>(p.conv_w + (int64_t)(c0 + i) * kConvTaps);
+      const uint32_t q[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < kConvTaps - 1; ++j) load_full(t0 + j, win[j]);
+      for (int k = 0; k < 2; ++k) {
+        w[0][i + k] = (double)__uint_as_float(q[2 * k] << 16);
+        w[1][i + k] = (double)__uint_as_float(q[2 * k] & 0xffff0000u);
+        w[2][i + k] = (double)__uint_as_float(q[2 * k + 1] << 16);
+        w[3][i + k] = (double)__uint_as_float(q[2 * k + 1] & 0xffff0000u);
+      }
+    }
+    uint32_t x[NW];
+    load_full(t0, x);
+    widen(x, wa);
+    load_full(t0 + 1, x);
+    widen(x, wb);
+    load_full(t0 + 2, x);
+    widen(x, wc);
+    load_full(t0 + kConvTaps - 1, xr[0]);
+    if (tn > 1) load_full(t0 + kConvTaps, xr[1]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      w[0][i] = w[1][i] = w[2][i] = w[3][i] = 0.0;
+      wa[i] = wb[i] = wc[i] = 0.0;
+    }
   }
-  // the new conv state is the 3 rows of [state ; tokens] that end at the last real token (rows len .. len + 2):
-  // the window after that token, or, for a sequence with no real token, the state's own window
-  if (p.conv_out && on && len == 0 && t0 == 0) {
+  // the new conv state is the 3 rows of [state ; tokens] that end at the last real token (rows len .. len + 2), written
+  // by the tile of that token (the first tile of a sequence with no real token)
+  if (p.conv_out && on && (len == 0 ? t0 == 0 : (len - 1) / kTok == t0 / kTok)) {
 #pragma unroll
-    for (int j = 0; j < kConvTaps - 1; ++j) store_raw(p.conv_out + (s * (kConvTaps - 1) + j) * p.C + c0, win[j]);
+    for (int j = 0; j < kConvTaps - 1; ++j) {
+      uint32_t x[NW];
+      load_full(len + j, x);
+#pragma unroll
+      for (int i = 0; i < NW; i += 4)
+        *reinterpret_cast<uint4*>(p.conv_out + (s * (kConvTaps - 1) + j) * p.C + c0 + 2 * i) =
+            make_uint4(x[i], x[i + 1], x[i + 2], x[i + 3]);
+    }
   }
 
-  // the next token's input row is loaded one token ahead, so its latency overlaps this token's work
-  uint32_t xn[kChan / 2];
-  if (on && tn > 0) load_full(t0 + kConvTaps - 1, xn);
-  for (int tt = 0; tt < tn; ++tt) {
+  const bool qk_chan = on && c0 < 2 * kd;
+  auto token = [&](int tt, const double (&x0)[NCH], const double (&x1)[NCH], const double (&x2)[NCH],
+                   double (&x3)[NCH], uint32_t (&raw)[NW]) {
     const int64_t t = t0 + tt, m = m_s + t;
-    float y[kChan];
-    if (on) {
-      uint32_t x[kChan / 2];
+    widen(raw, x3);
+    if (on && tt + 2 < tn) load_full(t + kConvTaps + 1, raw);
+    uint32_t yw[NW], gw[NW];
+    od_u16x2 far = {0, 0};  // the largest distance of 2 |g|'s pattern above the smallest that the table steps cover
 #pragma unroll
-      for (int i = 0; i < kChan / 2; ++i) x[i] = xn[i];
-      if (tt + 1 < tn) load_full(t + kConvTaps, xn);
+    for (int i = 0; i < NW; ++i) {
+      float acc[2];
 #pragma unroll
-      for (int i = 0; i < kChan; ++i) {
-        uint32_t w01 = wr[2 * i], w23 = wr[2 * i + 1];
-        // keeps the float64 taps out of the registers between tokens (hoisted, 64 doubles would take 128 VGPRs)
-        asm volatile("" : "+v"(w01), "+v"(w23));
-        double acc = (double)__uint_as_float(w01 << 16) * (double)chan(win[0], i);
-        acc += (double)__uint_as_float(w01 & 0xffff0000u) * (double)chan(win[1], i);
-        acc += (double)__uint_as_float(w23 << 16) * (double)chan(win[2], i);
-        acc += (double)__uint_as_float(w23 & 0xffff0000u) * (double)chan(x, i);
-        y[i] = silu_bf16(bf((float)acc));
+      for (int k = 0; k < 2; ++k) {  // exact products, so the fma chain rounds as separate float64 additions do
+        const int c = 2 * i + k;
+        acc[k] = (float)fma(w[3][c], x3[c], fma(w[2][c], x2[c], fma(w[1][c], x1[c], w[0][c] * x0[c])));
       }
+      const uint32_t g2 = od_pack_bf16x2(acc[0], acc[1]);
+      gw[i] = g2;
+      // bf16(silu(g)) of both halves: the table for 2^-8 <= |g| < 16, bf16(g / 2) (the pattern with the exponent one
+      // lower) for 2^-125 <= |g| below it
+      const od_u16x2 g = __builtin_bit_cast(od_u16x2, g2), d = g << 1;  // 2 |g|'s pattern
+      const od_u16x2 lo2 = {2 * kSiluLo, 2 * kSiluLo}, top = {2 * kSiluHalf - 2, 2 * kSiluHalf - 2};
+      const od_u16x2 at = (g >> 15) * (uint16_t)(2 * kSiluHalf) + __builtin_elementwise_min(__builtin_elementwise_sub_sat(d, lo2), top);
+      const uint32_t a2 = __builtin_bit_cast(uint32_t, at);
+      const char* tab = reinterpret_cast<const char*>(stab);
+      const uint32_t t2 = *reinterpret_cast<const uint16_t*>(tab + (a2 & 0xffffu)) |
+                          (uint32_t)*reinterpret_cast<const uint16_t*>(tab + (a2 >> 16)) << 16;
+      const od_u16x2 one = {1, 1}, below = (od_u16x2)0 - __builtin_elementwise_min(__builtin_elementwise_sub_sat(lo2, d), one);
+      const uint32_t m2 = __builtin_bit_cast(uint32_t, below);
+      yw[i] = (m2 & __builtin_bit_cast(uint32_t, (od_u16x2)(g - (uint16_t)0x80))) | (~m2 & t2);
+      far = __builtin_elementwise_max(far, (od_u16x2)(d - (uint16_t)0x200));
+    }
+    constexpr uint16_t kFar = 2 * kSiluHi - 0x200;  // |g| >= 16, infinite or NaN; |g| < 2^-125 wraps past it
+    if (__builtin_expect((far.x >= kFar || far.y >= kFar) && on, 0)) {
+      asm volatile("");  // a branch, not selects
 #pragma unroll
-      for (int i = 0; i < kChan / 2; ++i) {
-        win[0][i] = win[1][i];
-        win[1][i] = win[2][i];
-        win[2][i] = x[i];
-      }
-      if (p.conv_out && t == len - 1) {
-#pragma unroll
-        for (int j = 0; j < kConvTaps - 1; ++j) store_raw(p.conv_out + (s * (kConvTaps - 1) + j) * p.C + c0, win[j]);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kChan; ++i) y[i] = 0.0f;
+      for (int i = 0; i < NW; ++i)
+        yw[i] = od_pack_bf16x2(silu_bf16(__uint_as_float(gw[i] << 16)), silu_bf16(__uint_as_float(gw[i] & 0xffff0000u)));
     }
     // l2norm of the q and k heads: squares rounded to bf16, their exact sum rounded to bf16, + eps, rsqrt and the
     // product each rounded to bf16 (torch's bf16 arithmetic, with a correctly rounded rsqrt)
-    const bool qk_chan = on && c0 < 2 * kd;
-    double ss = 0.0;
-    if (qk_chan) {
+    if (__builtin_amdgcn_ballot_w64(qk_chan)) {
+      float y[NCH];
+      unpack(yw, y);
+      float ss = 0.0f;
+      float sq[NCH];
 #pragma unroll
-      for (int i = 0; i < kChan; ++i) ss += (double)bf(y[i] * y[i]);
-    }
-    for (int o = G / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, OD_WAVE);
-    if (qk_chan) {
-      const float sb = bf((float)ss);
-      const float den = bf(sb + 1e-6f);
-      const float inv = bf((float)(1.0 / sqrt((double)den)));
+      for (int i = 0; i < NCH; i += 2) {
+        sq[i] = y[i] * y[i];
+        sq[i + 1] = y[i + 1] * y[i + 1];
+        od_bfr2(sq[i], sq[i + 1]);
+        ss += sq[i] + sq[i + 1];
+      }
+      ss = group_sum(ss, G);
+      float sb = ss * (1.0f - 0x1p-20f), sh = ss * (1.0f + 0x1p-20f);
+      od_bfr2(sb, sh);
+      float den = bf(sb + 1e-6f);
+      float inv = __builtin_amdgcn_rsqf(den);
+      const bool slow = !(sb == sh) || ((__float_as_uint(inv) & 0xffffu) - 0x7ffcu) <= 8u;
+      if (__builtin_expect(__any(slow && qk_chan), 0)) {
+        double sd = 0.0;
 #pragma unroll
-      for (int i = 0; i < kChan; ++i) y[i] = bf(y[i] * inv);
-      store16(p.qk + m * (int64_t)(2 * kd) + c0, y);
-    } else if (on) {
-      store16(p.v + m * (int64_t)(p.n_v * p.dv) + (c0 - 2 * kd), y);
+        for (int i = 0; i < NCH; ++i) sd += (double)sq[i];
+        for (int o = G / 2; o > 0; o >>= 1) sd += __shfl_xor(sd, o, OD_WAVE);
+        den = bf(bf((float)sd) + 1e-6f);
+        inv = (float)(1.0 / sqrt((double)den));
+      }
+      inv = bf(inv);
+      if (qk_chan) {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) yw[i] = od_pack_bf16x2(y[2 * i] * inv, y[2 * i + 1] * inv);
+      }
     }
+    if (on) {
+      uint16_t* dst = qk_chan ? p.qk + m * (int64_t)(2 * kd) + c0 : p.v + m * (int64_t)(p.n_v * p.dv) + (c0 - 2 * kd);
+#pragma unroll
+      for (int i = 0; i < NW; i += 4)
+        *reinterpret_cast<uint4*>(dst + 2 * i) = make_uint4(yw[i], yw[i + 1], yw[i + 2], yw[i + 3]);
+    }
+  };
+  for (int tt = 0; tt < tn; tt += 4) {
+    token(tt, wa, wb, wc, wd, xr[0]);
+    if (tt + 1 >= tn) break;
+    token(tt + 1, wb, wc, wd, wa, xr[1]);
+    if (tt + 2 >= tn) break;
+    token(tt + 2, wc, wd, wa, wb, xr[0]);
+    if (tt + 3 >= tn) break;
+    token(tt + 3, wd, wa, wb, wc, xr[1]);
   }
 
   // gates of the tile's tokens (first channel block): thread i takes (token i / n_v, value head i % n_v). A right pad
@@ -567,9 +663,14 @@ extern "C" int od_gdn_prep_ex(const uint16_t* proj, int64_t ldp, const uint16_t*
   PrepArgs p{proj, conv_w, conv_in, seq_state, A_log, dt_bias, qk, v, g, beta, conv_out, seq_len, ldp, S, L,
              n_states, (int)n_k, (int)n_v, (int)dk, (int)dv, (int)C};
   const int64_t tiles = S * ((L + kTok - 1) / kTok);
-  const int64_t cblocks = (C / kChan + kPrepThreads - 1) / kPrepThreads;
-  gdn_prep_kernel<<<dim3((unsigned)tiles, (unsigned)cblocks), dim3(min(threads_for(C), kPrepThreads)), 0,
-                    (hipStream_t)stream>>>(p);
+  // 8 channels per thread (16-byte rows) wherever a head then fits a wave's lanes
+  const int nch = dk / 8 <= 64 ? 8 : 16;
+  const int threads = (int)min((C / nch + 63) / 64 * 64, (int64_t)kPrepThreads);
+  const dim3 grid((unsigned)tiles, (unsigned)((C / nch + threads - 1) / threads));
+  if (nch == 8)
+    gdn_prep_kernel<8><<<grid, dim3(threads), 0, (hipStream_t)stream>>>(p);
+  else
+    gdn_prep_kernel<16><<<grid, dim3(threads), 0, (hipStream_t)stream>>>(p);
   return od_launch_status();
 }
 

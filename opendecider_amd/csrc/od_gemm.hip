@@ -56,9 +56,6 @@ constexpr int kCpr = BK / 16;  // 16-byte chunks per row per stage
 constexpr int kGroupM = 4;
 constexpr int kScaleRows = 256;  // the WIDE variant's LDS scale slot: kScaleRows row scales, then 256 column scales
 constexpr int kOOB = 0x7ffffff0;  // a buffer offset past any range: the load returns zeros
-// The SwiGLU epilogue's LDS table of bf16(silu(g)) (od_silu_bf16) for 2^-8 <= |g| < 16: bf16 patterns
-// kSiluLo .. kSiluHi - 1 of each sign, positive ones first (2 x 1536 entries, 6 KB)
-constexpr uint32_t kSiluLo = 0x3b80u, kSiluHi = 0x4180u, kSiluHalf = kSiluHi - kSiluLo;
 
 struct GemmArgs {
   const int8_t* a;
@@ -447,11 +444,7 @@ __global__ __launch_bounds__(kThreads, BM == 128 && BN == 128 && NS == 2 ? 4 : 1
   // the wide SwiGLU epilogue's silu table, filled here (its first stage's barrier orders the fill before any read)
   __shared__ uint16_t stab[SWIGLU && WIDE ? 2 * kSiluHalf : 2];
   if constexpr (SWIGLU && WIDE) {
-    for (int i = threadIdx.x; i < (int)(2 * kSiluHalf); i += kThreads) {
-      const uint32_t h = (uint32_t)i >= kSiluHalf;
-      const uint32_t bits = (h << 15) | (kSiluLo + (uint32_t)i - h * kSiluHalf);
-      stab[i] = od_f32_to_bf16(od_silu_bf16(__uint_as_float(bits << 16)));
-    }
+    for (int i = threadIdx.x; i < (int)(2 * kSiluHalf); i += kThreads) stab[i] = od_silu_table_entry(i);
   }
 
   const int lane = threadIdx.x & 63;

@@ -63,6 +63,42 @@ def test_gdn_prep_bit_exact(gpu_lib, S, L, n_k, n_v, with_state):
     assert torch.equal(co.cpu(), new)
 
 
+@pytest.mark.parametrize("S,L,n_k,n_v,dk,dv", [(2, 15, 2, 4, 16, 32), (1, 16, 1, 2, 64, 128), (2, 17, 1, 1, 256, 64),
+                                               (1, 33, 1, 2, 512, 16), (1, 18, 1, 1, 1024, 16), (3, 32, 16, 32, 128, 128)])
+def test_gdn_prep_tiles_and_special_values(gpu_lib, S, L, n_k, n_v, dk, dv):
+    """od_gdn_prep at the edges of its 16-token tiles and over its head dims (2 to 64 lanes per head, 16 channels per
+    thread at 1024), inputs of every magnitude (zero rows, 2^-130 .. 2^120, sums at bf16 midpoints, infinities, NaN):
+    the oracle's bits, NaN for NaN."""
+    from opendecider_amd import kernels
+    g = torch.Generator().manual_seed(S * 100 + L + dk)
+    C = 2 * n_k * dk + n_v * dv
+    proj = _proj(g, S * L, n_k, n_v, dk, dv)
+    conv_w = _bf(g, C, 4, scale=0.3)
+    conv_w[::7] = 1.0                                             # exact sums: many ties
+    proj[L // 3, :C] = 0
+    scale = 2.0 ** torch.randint(-130, 121, (C,), generator=g).float()
+    proj[L // 2, :C] = (proj[L // 2, :C].float() * scale).to(torch.bfloat16)
+    proj[L - 1, 3] = float("inf")
+    proj[L - 1, 5] = float("-inf")
+    proj[L - 1, C - 2] = float("nan")
+    A_log = torch.log(torch.rand(n_v, generator=g) * 15.5 + 0.5).to(torch.bfloat16)
+    dt = (1 + 0.1 * torch.randn(n_v, generator=g)).to(torch.bfloat16)
+    conv_in = _bf(g, S, 3, C)
+    lens = torch.tensor([min(L, 16), L, 0][:S], dtype=torch.int32)
+    print(f"gdn_prep special S={S} L={L} dk={dk} dv={dv}", flush=True)
+    qk, v, _, _, co = kernels.gdn_prep(proj.to(DEV), conv_w.to(DEV), A_log.to(DEV), dt.to(DEV), S, L, n_k, n_v, dk, dv,
+                                       conv_in.to(DEV), conv_out=True, seq_len=lens.to(DEV))
+    cfg = og.GDNConfig(n_k_heads=n_k, n_v_heads=n_v, dk=dk, dv=dv)
+    y, new = og.conv_silu(og.split_proj(proj[:, :C + n_v * dv + 2 * n_v], cfg)[0].reshape(S, L, C), conv_w, conv_in, lens)
+    y = y.reshape(S * L, C)
+    kd = n_k * dk
+    want = torch.cat([og.l2norm_bf16(y[:, :kd].reshape(-1, n_k, dk)).reshape(-1, kd),
+                      og.l2norm_bf16(y[:, kd:2 * kd].reshape(-1, n_k, dk)).reshape(-1, kd)], 1)
+    for got, ref in ((qk.cpu(), want), (v.cpu(), y[:, 2 * kd:]), (co.cpu(), new)):  # (a NaN's payload is free)
+        assert torch.equal(got.isnan(), ref.isnan())
+        assert torch.equal(got.nan_to_num(nan=0.0).view(torch.int16), ref.nan_to_num(nan=0.0).view(torch.int16))
+
+
 @pytest.mark.parametrize("S,L,n_k,n_v,lens", [(4, 11, 2, 4, [11, 6, 2, 0]), (3, 40, 16, 32, [40, 17, 1]),
                                                (2, 9, 2, 4, [3, 8])])
 def test_gdn_prep_padded_sequences_bit_exact(gpu_lib, S, L, n_k, n_v, lens):
