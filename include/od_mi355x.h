@@ -539,6 +539,18 @@ int od_gdn_norm_quant(const uint16_t* o, int64_t ldo, const uint16_t* z, int64_t
                       const uint16_t* inv_s, float eps, int64_t M, int64_t n_v, int64_t dv, int8_t* xq, int64_t ldq,
                       float* sx, od_stream_t stream);
 
+/*
+ * Decision readout of the option rows (src/opendecider/v3.py:639-643,701-709, src/opendecider/decider.py:255-257):
+ *   h bf16 [B n_opt t, H] (row stride ldh), final_norm bf16 [H], head fp32 [H], none_logit fp32 [1]. Per token the final
+ *   RMSNorm hn = bf16(w * bf16(h * r)) (norm_offset: bf16((h * r) * (1 + w))), r as od_rmsnorm_quant takes it; per
+ *   option row the mean over its tokens t0 .. t - 1 of hn . head (float64 sums, rounded once) into logits fp32
+ *   [B n_opt] (a workspace of the caller); per request log_softmax([logits ; none_logit] * inv_temperature) into out
+ *   fp32 [B, n_opt + 1]. 0 <= t0 < t. Two launches.
+ */
+int od_readout(const uint16_t* h, int64_t ldh, const uint16_t* final_norm, int norm_offset, float eps,
+               const float* head, const float* none_logit, float inv_temperature, int64_t B, int64_t n_opt, int64_t t,
+               int64_t t0, int64_t H, float* logits, float* out, od_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

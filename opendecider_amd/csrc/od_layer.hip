@@ -472,6 +472,108 @@ void launch_silu_vec(dim3 grid, hipStream_t st, const uint16_t* gu, int64_t ldg,
   }
 }
 
+
+// ------------------------------------------------------------------------------------------------ readout
+struct ReadoutArgs {
+  const uint16_t* h;
+  const uint16_t* w;
+  const float* head;
+  const float* none;
+  float* logits;
+  float* out;
+  int64_t ldh, H;
+  int n_opt, t, t0, vec;
+  float eps, inv_temp;
+};
+
+// One workgroup per option row, its tokens shared out over the waves; a token's values are read twice (the sum of
+// squares, then the normed dot product: the second read hits the cache). Bound by the latency of those reads: one
+// launch over 32 MB in place of a dozen elementwise ones over float32 and float64 copies of it (4096 tokens x 4096:
+// about 250 -> 16 us).
+constexpr int kReadoutThreads = 256;
+template <bool OFFSET>
+__global__ __launch_bounds__(kReadoutThreads) void readout_rows_kernel(ReadoutArgs p) {
+  __shared__ double red[kReadoutThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double dot = 0.0;
+  for (int j = p.t0 + wave; j < p.t; j += kReadoutThreads / 64) {
+    const uint16_t* row = p.h + ((int64_t)blockIdx.x * p.t + j) * p.ldh;
+    double ss = 0.0;
+    const int64_t nv = p.vec ? p.H / 8 : 0;
+    for (int64_t c = lane; c < nv; c += 64) {
+      const uint4 x = *reinterpret_cast<const uint4*>(row + 8 * c);
+      const uint32_t xw[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double a = (double)__uint_as_float(xw[i] << 16), b = (double)__uint_as_float(xw[i] & 0xffff0000u);
+        ss = fma(a, a, ss);
+        ss = fma(b, b, ss);
+      }
+    }
+    for (int64_t c = 8 * nv + lane; c < p.H; c += 64) {
+      const double a = (double)od_bf16_to_f32(row[c]);
+      ss = fma(a, a, ss);
+    }
+    const float r = od_rms_factor(od_group_sum_f64<64>(ss), p.H, p.eps);
+    auto normed = [&](float x, float w) {
+      float y = x * r;
+      if (OFFSET) return od_bf16_to_f32(od_f32_to_bf16(y * (1.0f + w)));
+      return od_bf16_to_f32(od_f32_to_bf16(w * od_bf16_to_f32(od_f32_to_bf16(y))));
+    };
+    for (int64_t c = lane; c < nv; c += 64) {
+      const uint4 x = *reinterpret_cast<const uint4*>(row + 8 * c), w = *reinterpret_cast<const uint4*>(p.w + 8 * c);
+      const float4 a0 = *reinterpret_cast<const float4*>(p.head + 8 * c);
+      const float4 a1 = *reinterpret_cast<const float4*>(p.head + 8 * c + 4);
+      const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, ww[4] = {w.x, w.y, w.z, w.w};
+      const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dot = fma((double)normed(__uint_as_float(xw[i] << 16), __uint_as_float(ww[i] << 16)), (double)av[2 * i], dot);
+        dot = fma((double)normed(__uint_as_float(xw[i] & 0xffff0000u), __uint_as_float(ww[i] & 0xffff0000u)),
+                  (double)av[2 * i + 1], dot);
+      }
+    }
+    for (int64_t c = 8 * nv + lane; c < p.H; c += 64)
+      dot = fma((double)normed(od_bf16_to_f32(row[c]), od_bf16_to_f32(p.w[c])), (double)p.head[c], dot);
+  }
+  dot = od_group_sum_f64<64>(dot);
+  if (lane == 0) red[wave] = dot;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < kReadoutThreads / 64; ++i) s += red[i];
+    p.logits[blockIdx.x] = (float)(s / (double)(p.t - p.t0));
+  }
+}
+
+// log_softmax over a request's option logits and the none logit, one workgroup per request
+__global__ __launch_bounds__(kReadoutThreads) void readout_softmax_kernel(ReadoutArgs p) {
+  __shared__ float red[kReadoutThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = p.n_opt + 1;
+  const float* x = p.logits + (int64_t)blockIdx.x * p.n_opt;
+  auto value = [&](int i) { return (i < p.n_opt ? x[i] : p.none[0]) * p.inv_temp; };
+  auto reduce = [&](float v, bool mx) {
+    for (int o = 32; o > 0; o >>= 1) {
+      const float y = __shfl_xor(v, o, OD_WAVE);
+      v = mx ? fmaxf(v, y) : v + y;
+    }
+    __syncthreads();
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    v = red[0];
+    for (int i = 1; i < kReadoutThreads / 64; ++i) v = mx ? fmaxf(v, red[i]) : v + red[i];
+    return v;
+  };
+  float m = -INFINITY;
+  for (int i = threadIdx.x; i < n; i += kReadoutThreads) m = fmaxf(m, value(i));  // (a NaN comes back through the sum)
+  m = reduce(m, true);
+  float s = 0.0f;
+  for (int i = threadIdx.x; i < n; i += kReadoutThreads) s += expf(value(i) - m);
+  const float lse = logf(reduce(s, false));
+  for (int i = threadIdx.x; i < n; i += kReadoutThreads) p.out[(int64_t)blockIdx.x * n + i] = value(i) - m - lse;
+}
+
 }  // namespace
 
 extern "C" int od_rmsnorm_quant_ex(const uint16_t* x, int64_t ldx, const uint16_t* w, const uint16_t* inv_s,
@@ -657,4 +759,26 @@ extern "C" int od_qk_norm_rope_kv_append(uint16_t* qkv, int64_t ld, int64_t B, i
   if (D != 64 && D != 128) return OD_ERR_UNSUPPORTED;
   return od_qk_norm_rope_kv_append_ex(qkv, ld, B, S, n_heads_q, n_heads_k, D, D, 0, q_w, k_w, cos_t, sin_t, n_pos,
                                       pos, eps, kq, ks, vq, vs, cap, n0, stream);
+}
+
+extern "C" int od_readout(const uint16_t* h, int64_t ldh, const uint16_t* final_norm, int norm_offset, float eps,
+                          const float* head, const float* none_logit, float inv_temperature, int64_t B, int64_t n_opt,
+                          int64_t t, int64_t t0, int64_t H, float* logits, float* out, od_stream_t stream) {
+  if (B < 0 || n_opt < 0 || H < 1 || t < 1 || t0 < 0 || t0 >= t || ldh < H) return OD_ERR_SHAPE;
+  if (B == 0) return OD_OK;
+  if (!none_logit || !out) return OD_ERR_NULL;
+  if (n_opt > 0 && (!h || !final_norm || !head || !logits)) return OD_ERR_NULL;
+  if (B * n_opt > 0x7fffffffll || B > 0x7fffffffll || n_opt >= 0x7fffffffll || t > 0x7fffffffll) return OD_ERR_SHAPE;
+  ReadoutArgs p{h, final_norm, head, none_logit, logits, out, ldh, H, (int)n_opt, (int)t, (int)t0,
+                ldh % 8 == 0 && od_aligned16(h) && od_aligned16(final_norm) && od_aligned16(head) ? 1 : 0, eps,
+                inv_temperature};
+  hipStream_t st = (hipStream_t)stream;
+  if (n_opt > 0) {
+    if (norm_offset)
+      readout_rows_kernel<true><<<dim3((unsigned)(B * n_opt)), dim3(kReadoutThreads), 0, st>>>(p);
+    else
+      readout_rows_kernel<false><<<dim3((unsigned)(B * n_opt)), dim3(kReadoutThreads), 0, st>>>(p);
+  }
+  readout_softmax_kernel<<<dim3((unsigned)B), dim3(kReadoutThreads), 0, st>>>(p);
+  return od_launch_status();
 }

@@ -465,7 +465,7 @@ class DenseDecoder:
                 conv_tmp = self._conv_tmp(B)
         ws = self.workspace(B * S)
         h, mid = ws["h"]
-        h.copy_(self.embed.index_select(0, ids.reshape(-1)))
+        self._embed(ids)
         pos, row_start = self.prefill_layout(n0, B, S)
         for li in range(len(self.layers)):
             if self.layers[li]["gdn"]:
@@ -476,6 +476,13 @@ class DenseDecoder:
             if isinstance(st, GDNState):
                 st.length = n0 + S
         return h
+
+    def _embed(self, ids: torch.Tensor) -> torch.Tensor:
+        """The tokens' embeddings, gathered straight into the residual buffer of their workspace (returned)."""
+        h = self.workspace(ids.numel())["h"][0]
+        if self.embed.dtype == h.dtype and not self.embed.requires_grad:
+            return torch.index_select(self.embed, 0, ids.reshape(-1), out=h)
+        return h.copy_(self.embed.index_select(0, ids.reshape(-1)))
 
     def _conv_tmp(self, B: int) -> torch.Tensor:
         key = ("conv_tmp", B)
@@ -501,7 +508,8 @@ class DenseDecoder:
             raise ValueError("rows_forward: GDN layers need row_state and take no key mask")
         ws = self.workspace(h0.shape[0])
         h, mid = ws["h"]
-        h.copy_(h0)
+        if h0 is not h:
+            h.copy_(h0)
         for li in range(len(self.layers)):
             if self.layers[li]["gdn"]:
                 self.gdn_layer(li, h, mid, ws, states[li], R, t, row_state)
@@ -535,7 +543,7 @@ class DenseDecoder:
             raise ValueError(f"question_pass: group_state outside [0, {Ns})")
         ws = self.workspace(G * Lq)
         h, mid = ws["h"]
-        h.copy_(self.embed.index_select(0, ids_q.reshape(-1)))
+        self._embed(ids_q)
         pos = (T + torch.arange(Lq, dtype=torch.int32)).repeat(G).to(self.dev)
         row_start, max_rows = kernels.row_start_of([gs.count(s) for s in range(Ns)], self.dev)
         qmask = (torch.arange(Lq)[None, :] < torch.tensor(qlen)[:, None]).to(torch.uint8).to(self.dev)
@@ -589,7 +597,7 @@ class DenseDecoder:
         pos, row_start, max_rows, row_q = self._rows[key]
         ws = self.workspace(R * t)
         h, mid = ws["h"]
-        h.copy_(self.embed.index_select(0, ids_o.reshape(-1)))
+        self._embed(ids_o)
         Ns = self.state_count(states)
         D = cfg.head_dim
         for li in range(len(self.layers)):
@@ -613,6 +621,13 @@ class DenseDecoder:
         divided by the decision temperature (softmax(logits / T), decider.py:255-257), log-softmax per request:
         (B, n_opt + 1) fp32. The RMSNorm factor is the correctly rounded one (a float64 mean of squares, as
         od_rmsnorm_quant computes it); with cfg.norm_offset the zero-centred norm bf16((h * r) * (1 + w))."""
+        params = (h, self.final_norm, self.head, self.none_logit)
+        if h.dtype == self.final_norm.dtype == torch.bfloat16 and h.is_cuda and h.dim() == 2 and h.stride(1) == 1 \
+                and self.temperature != 0 and not (torch.is_grad_enabled() and any(x.requires_grad for x in params)):
+            t0, t1, _ = slice(0 if pool_last is None else t - pool_last, None).indices(t)
+            if t0 < t1:
+                return kernels.readout(h, self.final_norm, self.head, self.none_logit, self._eps32, self.temperature, B,
+                                       n_opt, t, t0, self.cfg.norm_offset)
         hf = h.float()
         hd = hf.double()
         r = (1.0 / torch.sqrt((hd * hd).sum(-1, keepdim=True) / hd.shape[-1] + self._eps32)).float()
@@ -636,7 +651,7 @@ class DenseDecoder:
         B, n_opt, t = ids.shape
         R = B * n_opt
         T = self.state_length(states)
-        h0 = self.embed.index_select(0, ids.reshape(-1))
+        h0 = self._embed(ids)
         pos, row_start, max_rows = self.row_layout(T, B, n_opt, t)
         h = self.rows_forward(h0, states, R, t, pos, row_start, max_rows, kvalid, self.row_states(B, n_opt))
         return self.readout(h, B, n_opt, t, pool_last)

@@ -712,6 +712,26 @@ def wide_attn(q, k, v, scale: float, kvalid=None, causal: bool = True, return_ls
     return (out, lse) if return_lse else out
 
 
+def readout(h: torch.Tensor, final_norm: torch.Tensor, head: torch.Tensor, none_logit: torch.Tensor, eps: float,
+            temperature: float, B: int, n_opt: int, t: int, t0: int = 0, offset: bool = False) -> torch.Tensor:
+    """od_readout: h (B n_opt t, H) bf16 with contiguous rows, final_norm (H,) bf16, head (H,) fp32, none_logit () fp32.
+    log_softmax over each request's option logits (the mean over an option's tokens t0 .. t - 1 of the normed hidden
+    state times head) and the none logit, divided by the temperature: (B, n_opt + 1) fp32."""
+    require_gpu(h, final_norm, head, none_logit, name="readout")
+    _lib.bf16_bits(h)
+    H = h.shape[-1]
+    if h.dim() != 2 or h.shape[0] != B * n_opt * t or h.stride(1) != 1:
+        raise ValueError("readout: h must be (B n_opt t, H) with contiguous rows")
+    final_norm = _vec(final_norm, H, "final_norm")
+    head, none_logit = _scales(head, H, "head"), _scales(none_logit, 1, "none_logit")
+    logits = torch.empty(max(B * n_opt, 1), dtype=torch.float32, device=h.device)
+    out = torch.empty(B, n_opt + 1, dtype=torch.float32, device=h.device)
+    check(lib().od_readout(ptr(h), h.stride(0) if h.shape[0] > 1 else H, ptr(final_norm), int(bool(offset)), float(eps),
+                           ptr(head), ptr(none_logit), 1.0 / float(temperature), B, n_opt, t, t0, H, ptr(logits),
+                           ptr(out), stream_of(h)), "od_readout")
+    return out
+
+
 def _lm_h_operands(h: torch.Tensor, K: int):
     """(hb bf16 rows for the matmul, hn rows for the target term, hn_fp32 flag, M, leading shape)."""
     if h.shape[-1] != K:

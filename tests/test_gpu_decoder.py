@@ -305,6 +305,28 @@ def test_decoder_layers_stage_by_stage(gpu_lib, name, cfg_kw, B, n_opt, t, T):
     assert (lp.cpu() - ref).abs().max().item() <= 1e-6, "readout"
 
 
+@pytest.mark.parametrize("B,n_opt,t,t0,H,offset,pad", [(1, 1, 1, 0, 8, False, 0), (3, 5, 4, 0, 100, False, 0),
+                                                       (2, 300, 2, 1, 256, True, 0), (2, 3, 9, 6, 4096, False, 0),
+                                                       (1, 2, 24, 0, 1028, True, 4), (2, 0, 3, 0, 64, False, 0)])
+def test_readout_kernel(gpu_lib, B, n_opt, t, t0, H, offset, pad):
+    """od_readout against float64 on the oracle's normed rows: widths with and without 16-byte rows, one token to more
+    than the waves of a workgroup, a token range, more options than threads, no options at all. Sums are float64, so
+    what is left is the fp32 rounding of the logits and of log_softmax: a few 2^-24 of the largest value."""
+    from opendecider_amd import kernels
+    g = torch.Generator().manual_seed(B * 100 + H + t)
+    big = torch.randn(B * n_opt * t, H + pad, generator=g).to(torch.bfloat16).to(DEV)
+    h = big[:, pad:]
+    w = ((0.0 if offset else 1.0) + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16)
+    head, none = torch.randn(H, generator=g) / H ** 0.5, torch.tensor(0.3)
+    print(f"readout B={B} n_opt={n_opt} t={t} t0={t0} H={H} offset={offset}", flush=True)
+    got = kernels.readout(h, w.to(DEV), head.to(DEV), none.to(DEV), 1e-6, 0.7, B, n_opt, t, t0, offset).cpu()
+    hn = od.rmsnorm(h.cpu(), w, 1e-6, offset).double().reshape(B, n_opt, t, H)[:, :, t0:].mean(2)
+    logits = torch.cat([hn @ head.double(), none.double().expand(B, 1)], 1) / 0.7
+    ref = torch.log_softmax(logits, -1)
+    assert got.shape == ref.shape
+    assert (got - ref).abs().max().item() <= 2.0 ** -21 * max(1.0, ref.abs().max().item())
+
+
 T1_MULTIPLE = 2.0
 
 
