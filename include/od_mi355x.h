@@ -540,6 +540,15 @@ int od_gdn_norm_quant(const uint16_t* o, int64_t ldo, const uint16_t* z, int64_t
                       float* sx, od_stream_t stream);
 
 /*
+ * A W8A8 linear in one call: od_act_quant of x bf16 [M, ldx] (inv_s as there) into xq int8 [M, K] and sx fp32 [M]
+ * (workspaces of the caller, xq 16-byte aligned), then od_w8a8_gemm_ws over them (ws / ws_ints as there; NULL and 0 for
+ * shapes that it does not split): out bf16 [M, ldo]. K % 16 == 0. The same launches and the same bytes as the two calls.
+ */
+int od_w8a8_linear(const uint16_t* x, int64_t ldx, const uint16_t* inv_s, const int8_t* w, int64_t ldw, const float* sw,
+                   const uint16_t* bias, const uint16_t* residual, int64_t ldr, uint16_t* out, int64_t ldo, int8_t* xq,
+                   float* sx, int64_t M, int64_t N, int64_t K, int32_t* ws, int64_t ws_ints, od_stream_t stream);
+
+/*
  * Decision readout of the option rows (src/opendecider/v3.py:639-643,701-709, src/opendecider/decider.py:255-257):
  *   h bf16 [B n_opt t, H] (row stride ldh), final_norm bf16 [H], head fp32 [H], none_logit fp32 [1]. Per token the final
  *   RMSNorm hn = bf16(w * bf16(h * r)) (norm_offset: bf16((h * r) * (1 + w))), r as od_rmsnorm_quant takes it; per

@@ -1162,3 +1162,17 @@ extern "C" int od_w8a8_gemm_ws(const int8_t* a, int64_t lda, const float* sa, co
   const bool split = sp.splits > 1 && ws && ws_ints >= sp.ws_ints && od_aligned16(ws);
   return gemm_launch(p, swiglu != 0, (hipStream_t)stream, split ? &sp : nullptr, split ? ws : nullptr);
 }
+
+extern "C" int od_w8a8_linear(const uint16_t* x, int64_t ldx, const uint16_t* inv_s, const int8_t* w, int64_t ldw,
+                              const float* sw, const uint16_t* bias, const uint16_t* residual, int64_t ldr,
+                              uint16_t* out, int64_t ldo, int8_t* xq, float* sx, int64_t M, int64_t N, int64_t K,
+                              int32_t* ws, int64_t ws_ints, od_stream_t stream) {
+  if (M < 0 || N < 0 || K < 1 || ldw < K || ldo < N || (residual && ldr < N)) return OD_ERR_SHAPE;
+  if (M == 0 || N == 0) return OD_OK;
+  if (!w || !sw || !out || !xq || !sx) return OD_ERR_NULL;
+  int rc = gemm_check(xq, K, w, ldw, K);
+  if (rc != OD_OK) return rc;
+  rc = od_act_quant(x, ldx, inv_s, xq, K, sx, M, K, stream);
+  if (rc != OD_OK) return rc;
+  return od_w8a8_gemm_ws(xq, K, sx, w, ldw, sw, bias, residual, ldr, out, ldo, M, N, K, 0, ws, ws_ints, stream);
+}

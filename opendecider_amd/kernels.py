@@ -220,6 +220,8 @@ def splitk_workspace(M: int, N: int, Kp: int, device) -> torch.Tensor | None:
     key = (device.index, M, N, Kp)
     n = _SPLITK_WS.get(key)
     if n is None:
+        if len(_SPLITK_WS) >= 65536:  # the sizes are cheap to ask for again
+            _SPLITK_WS.clear()
         v = ctypes.c_int64(0)
         with torch.cuda.device(device):
             check(lib().od_w8a8_gemm_ws_size(M, N, Kp, ctypes.byref(v)), "od_w8a8_gemm_ws_size")
@@ -264,6 +266,42 @@ def w8a8_gemm(a: torch.Tensor, sa: torch.Tensor, w: torch.Tensor, sw: torch.Tens
     if want_acc:
         return o, acc
     return o
+
+
+def w8a8_linear(x: torch.Tensor, w: torch.Tensor, sw: torch.Tensor, bias=None, inv_s=None, in_features: int | None = None,
+                residual=None) -> torch.Tensor:
+    """act_quant and w8a8_gemm of x (..., in_features) bf16 with int8 w (N, Kp): (..., N) bf16, the same bytes. One call
+    into the library where the rows need no padding (Kp == in_features): a small linear is bound by the host, and the
+    two wrappers with their buffers took 25 us of it (M = 64, 2048 -> 6144; the kernels 10)."""
+    K = w.shape[1] if in_features is None else in_features
+    N, Kp = w.shape
+    if Kp != K or x.shape[-1] != K:
+        xq, sx = act_quant(x, inv_s, ld=Kp)
+        return w8a8_gemm(xq, sx, w, sw, bias, residual).view(*x.shape[:-1], N)
+    require_gpu(x, w, sw, bias, inv_s, residual, name="w8a8_linear")
+    _lib.bf16_bits(x)
+    if w.dtype != torch.int8:
+        raise TypeError("w8a8_linear: w must be int8")
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
+    if x2.stride(1) != 1:
+        x2 = x2.contiguous()
+    M, dev = x2.shape[0], x.device
+    inv_s, sw = _vec(inv_s, K, "inv_s"), _scales(sw, N, "w8a8_linear: sw")
+    if residual is not None:
+        _lib.bf16_bits(residual)
+        if residual.shape != (M, N) or residual.stride(-1) != 1:
+            raise ValueError("w8a8_linear: residual must be (M, N) with contiguous rows")
+    if bias is not None:
+        bias = _lib.bf16_bits(bias).contiguous()
+    buf = torch.empty(M * (K + 4), dtype=torch.int8, device=dev)  # quantized rows, then their fp32 scales
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    ws = splitk_workspace(M, N, K, dev)
+    xq = buf.data_ptr()
+    check(lib().od_w8a8_linear(x2.data_ptr(), x2.stride(0) if M > 1 else K, ptr(inv_s), w.data_ptr(), w.stride(0),
+                               sw.data_ptr(), ptr(bias), ptr(residual), 0 if residual is None else residual.stride(0),
+                               out.data_ptr(), N, xq, xq + M * K, M, N, K, ptr(ws), 0 if ws is None else ws.numel(),
+                               stream_of(x)), "od_w8a8_linear")
+    return out if x.dim() == 2 else out.view(*x.shape[:-1], N)
 
 
 def interleave_gate_up(w: torch.Tensor) -> torch.Tensor:

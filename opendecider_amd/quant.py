@@ -206,12 +206,9 @@ class W8A8Linear(nn.Module):
     def forward(self, x: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
         if not x.is_cuda:
             raise RuntimeError("W8A8Linear runs on the MI355X only (no CPU path)")
-        lead = x.shape[:-1]
         xb = x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16)
-        xq, sx = kernels.act_quant(xb, self.inv_s, ld=self.qweight.shape[1])
         res = None if residual is None else residual.reshape(-1, self.out_features)
-        y = kernels.w8a8_gemm(xq, sx, self.qweight, self.w_scale, self.bias, res)
-        y = y.view(*lead, self.out_features)
+        y = kernels.w8a8_linear(xb, self.qweight, self.w_scale, self.bias, self.inv_s, self.in_features, res)
         return y if x.dtype == torch.bfloat16 else y.to(x.dtype)
 
     def extra_repr(self) -> str:

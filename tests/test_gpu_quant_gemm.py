@@ -520,3 +520,33 @@ def test_splitk_bit_identical_to_one_pass(gpu_lib, M, N, K, epi):
         refo = oq.w8a8_epilogue(oq.int_gemm(a, w), sa, sw, None if bias is None else bias.cpu(),
                                 None if res is None else res.cpu())
         assert torch.equal(got.cpu(), refo)
+
+
+@pytest.mark.parametrize("shape,N,K,smooth,bias,residual", [((1,), 64, 16, False, False, False), ((7,), 6144, 2048, True, True, True),
+                                                           ((3, 5), 200, 48, True, False, True), ((2, 3, 4), 33, 100, False, True, False),
+                                                           ((600,), 6144, 2048, False, False, False), ((0,), 64, 32, False, True, False),
+                                                           ((), 40, 64, True, True, False)])
+def test_w8a8_linear_one_call_equals_two(gpu_lib, shape, N, K, smooth, bias, residual):
+    """W8A8Linear's one library call gives the bytes of act_quant and w8a8_gemm: leading shapes of every rank (none
+    and empty too), rows that need padding (K = 100) and strided ones, a shape that splits K, bias and residual."""
+    from opendecider_amd import kernels
+    from opendecider_amd.quant import W8A8Linear
+    g = torch.Generator().manual_seed(N + K)
+    big = torch.randn(*shape, K + 16, generator=g).to(torch.bfloat16).to(DEV)
+    x = big[..., 8:8 + K]
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(DEV)
+    sw = torch.rand(N, generator=g).to(DEV) * 1e-2
+    inv = (torch.rand(K, generator=g) + 0.5).to(torch.bfloat16).to(DEV) if smooth else None
+    b = torch.randn(N, generator=g).to(torch.bfloat16).to(DEV) if bias else None
+    res = torch.randn(*shape, N, generator=g).to(torch.bfloat16).to(DEV) if residual else None
+    m = W8A8Linear(w, sw, b, K, inv)
+    print(f"w8a8_linear {shape} N={N} K={K}", flush=True)
+    got = m(x, res)
+    xq, sx = kernels.act_quant(x, inv, ld=m.qweight.shape[1])
+    ref = kernels.w8a8_gemm(xq, sx, m.qweight, m.w_scale, m.bias, None if res is None else res.reshape(-1, N))
+    assert got.shape == (*shape, N) and torch.equal(got, ref.view(*shape, N))
+    if shape and shape[0]:
+        with pytest.raises((ValueError, RuntimeError)):  # more features than the layer has
+            m(big)
+    with pytest.raises(RuntimeError):
+        m(x.cpu())
