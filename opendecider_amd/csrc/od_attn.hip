@@ -884,6 +884,9 @@ __device__ __forceinline__ void own_stage(const AttnArgs& p, float (&red)[2][kWa
   bi.masked = 0;  // the causal mask is applied per score
 }
 
+// A barrier over LDS that leaves global loads in flight
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // DV: the value columns one workgroup accumulates (D, or D / 2 at D = 256: the two halves of a slot tile are two
 // workgroups, each recomputing the same scores and softmax; see branched_launch).
 template <int D, int DV, bool STAGED>
@@ -1003,24 +1006,25 @@ __device__ __forceinline__ void branched_attn_body(const AttnArgs& p, Smem<D>& s
         if (b + 1 < b_hi) step(b + 1, s1, s0);
       }
     } else {
-      // the int8 state, converted here: registers first (loads issued during the previous block), then LDS
+      // the int8 state, converted here: registers first, then LDS. A block is loaded right after the block before it is
+      // converted, a whole step ahead of its own conversion: issued between the softmax and the P.V product of the
+      // same step, the conversion waited for most of the memory latency (8 states x 32768 keys, 128 slots per head: 271
+      // -> 256 us; bound now by its 587 vector instructions per block and wave, half of them the conversion)
       const PrefixSrc src = prefix_src<D>(p.kq, p.ks, p.vq, p.vs, p.kvalid, p.Hkv, p.T, p.cap, s, g);
       PrefixRegs<D> pr;
       prefix_load<D>(src, p.T, b_lo * kBlockKeys, pr);
       BlockInfo cur = convert_block<D>(pr, sm.b[0], p.scale_log2, p.dq);
-      __syncthreads();
+      prefix_load<D>(src, p.T, min(b_lo + 1, b_hi - 1) * kBlockKeys, pr);
+      lds_barrier();
       for (int b = b_lo; b < b_hi; ++b) {
         const int buf = (b - b_lo) & 1;
         const BlockImg<D>& bk = sm.b[buf];
         attend_block<D, DV, 2, false>(bk.k, bk.vt + vcol, bk.gk, bk.kb, qf, 0.0f, cur.eb, cur.masked != 0, m_run,
-                                      l_run, e_run, o,
-                                  0, 0, slot_row, slot_tok, [&] {
-                                    if (b + 1 < b_hi) prefix_load<D>(src, p.T, (b + 1) * kBlockKeys, pr);
-                                  });
-        BlockInfo nxt = cur;
-        if (b + 1 < b_hi) nxt = convert_block<D>(pr, sm.b[buf ^ 1], p.scale_log2, p.dq);
-        __syncthreads();
-        cur = nxt;
+                                      l_run, e_run, o, 0, 0, slot_row, slot_tok, [] {});
+        if (b + 1 >= b_hi) break;
+        cur = convert_block<D>(pr, sm.b[buf ^ 1], p.scale_log2, p.dq);
+        prefix_load<D>(src, p.T, min(b + 2, b_hi - 1) * kBlockKeys, pr);
+        lds_barrier();
       }
     }
   }
