@@ -2,7 +2,8 @@
  * od_mi355x.h — C ABI of the MI355X (gfx950) kernels for OpenDecider's quantized scoring forward path.
  *
  * Conventions (all entry points):
- *   - Pointers are DEVICE pointers of the current HIP device; bf16 tensors are passed as uint16_t bit patterns.
+ *   - Pointers are DEVICE pointers of the current HIP device (but for parameters named host_*); bf16 tensors are
+ *     passed as uint16_t bit patterns.
  *   - Sizes and strides are in ELEMENTS, int64_t; the last dimension of every tensor is contiguous.
  *   - `stream` is a hipStream_t passed as void* (NULL = the legacy default stream). Work is enqueued on it and
  *     the call returns without synchronizing.
@@ -538,6 +539,12 @@ int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, const float
 int od_gdn_norm_quant(const uint16_t* o, int64_t ldo, const uint16_t* z, int64_t ldz, const uint16_t* w,
                       const uint16_t* inv_s, float eps, int64_t M, int64_t n_v, int64_t dv, int8_t* xq, int64_t ldq,
                       float* sx, od_stream_t stream);
+
+/*
+ * n int32 values from HOST memory (read during the call) into device memory, as kernel arguments: row offsets and
+ * other small tables without a host-to-device copy (which waits for the stream where the host memory is pageable).
+ */
+int od_fill_i32(const int32_t* host_values, int64_t n, int32_t* out, od_stream_t stream);
 
 /*
  * A W8A8 linear in one call: od_act_quant of x bf16 [M, ldx] (inv_s as there) into xq int8 [M, K] and sx fp32 [M]

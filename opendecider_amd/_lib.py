@@ -86,6 +86,7 @@ SIGNATURES = {
     "od_gdn_chunk_ws_size": [_i64, _i64, _i64, _c_ptr],
     "od_gdn_recurrence_chunked": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _i64, _c_ptr, _c_ptr, _c_ptr, _i64, _c_ptr],
+    "od_fill_i32": [_c_ptr, _i64, _c_ptr, _c_ptr],
     "od_w8a8_linear": [_c_ptr, _i64, _c_ptr, _c_ptr, _i64, _c_ptr, _c_ptr, _c_ptr, _i64, _c_ptr, _i64, _c_ptr, _c_ptr,
                        _i64, _i64, _i64, _c_ptr, _i64, _c_ptr],
     "od_readout": [_c_ptr, _i64, _c_ptr, ctypes.c_int, ctypes.c_float, _c_ptr, _c_ptr, ctypes.c_float, _i64, _i64, _i64,

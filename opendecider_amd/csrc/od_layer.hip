@@ -574,6 +574,18 @@ __global__ __launch_bounds__(kReadoutThreads) void readout_softmax_kernel(Readou
   for (int i = threadIdx.x; i < n; i += kReadoutThreads) p.out[(int64_t)blockIdx.x * n + i] = value(i) - m - lse;
 }
 
+
+// ------------------------------------------------------------------------------------------------ small tables
+constexpr int kFillValues = 512;  // 2 KB of kernel arguments
+struct FillArgs {
+  int32_t v[kFillValues];
+  int32_t* out;
+  int n;
+};
+__global__ __launch_bounds__(64) void fill_i32_kernel(FillArgs p) {
+  for (int i = threadIdx.x; i < p.n; i += 64) p.out[i] = p.v[i];
+}
+
 }  // namespace
 
 extern "C" int od_rmsnorm_quant_ex(const uint16_t* x, int64_t ldx, const uint16_t* w, const uint16_t* inv_s,
@@ -780,5 +792,20 @@ extern "C" int od_readout(const uint16_t* h, int64_t ldh, const uint16_t* final_
       readout_rows_kernel<false><<<dim3((unsigned)(B * n_opt)), dim3(kReadoutThreads), 0, st>>>(p);
   }
   readout_softmax_kernel<<<dim3((unsigned)B), dim3(kReadoutThreads), 0, st>>>(p);
+  return od_launch_status();
+}
+
+extern "C" int od_fill_i32(const int32_t* host_values, int64_t n, int32_t* out, od_stream_t stream) {
+  if (n < 0) return OD_ERR_SHAPE;
+  if (n == 0) return OD_OK;
+  if (!host_values || !out) return OD_ERR_NULL;
+  FillArgs p;
+  for (int64_t i = 0; i < n; i += kFillValues) {
+    p.n = (int)(n - i < kFillValues ? n - i : kFillValues);
+    p.out = out + i;
+    for (int k = 0; k < p.n; ++k) p.v[k] = host_values[i + k];
+    for (int k = p.n; k < kFillValues; ++k) p.v[k] = 0;
+    fill_i32_kernel<<<dim3(1), dim3(64), 0, (hipStream_t)stream>>>(p);
+  }
   return od_launch_status();
 }

@@ -400,7 +400,14 @@ def row_start_of(row_counts, device) -> tuple[torch.Tensor, int]:
     starts = [0]
     for c in counts:
         starts.append(starts[-1] + c)
-    return torch.tensor(starts, dtype=torch.int32).to(device, non_blocking=True), max(counts)
+    device = torch.device(device)
+    if device.type != "cuda" or device.index not in (None, torch.cuda.current_device()) or starts[-1] > 0x7fffffff:
+        return torch.tensor(starts, dtype=torch.int32).to(device, non_blocking=True), max(counts)
+    # as kernel arguments: a copy from pageable memory costs the host more and waits for the stream's earlier work
+    out = torch.empty(len(starts), dtype=torch.int32, device=device)
+    check(lib().od_fill_i32((ctypes.c_int32 * len(starts))(*starts), len(starts), out.data_ptr(), stream_of(out)),
+          "od_fill_i32")
+    return out, max(counts)
 
 
 def split_count(slot_tiles: int, T: int, n_cu: int = 256, wg_per_cu: int = 2, min_blocks: int = 4) -> int:

@@ -322,3 +322,29 @@ def test_two_level_without_questions_equals_one_level(gpu_lib):
     ref, ref_lse = run_gpu(c, staged=True, n_split=1)
     out, lse = _run_two_level(c, None, None, None, torch.arange(2, dtype=torch.int32), [3, 4], 260, 0, n_split=1)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16)) and torch.equal(lse, ref_lse)
+
+
+@pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 1400])
+def test_row_offsets_without_a_copy(gpu_lib, n):
+    """row_start_of's device offsets (kernel arguments, 512 per launch) are the running sums, also behind other work on
+    a side stream and inside a captured graph."""
+    from opendecider_amd import kernels
+    counts = [(7 * i) % 5 for i in range(n)]
+    want = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    print(f"row offsets n={n}", flush=True)
+    got, mx = kernels.row_start_of(counts, DEV)
+    assert got.dtype == torch.int32 and torch.equal(got.cpu(), want) and mx == max(counts)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.randn(1 << 20, device=DEV).sort()
+        got, _ = kernels.row_start_of(counts, DEV)
+    side.synchronize()
+    assert torch.equal(got.cpu(), want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        got, _ = kernels.row_start_of(counts, DEV)
+    for _ in range(3):
+        got.fill_(-1)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.cpu(), want)
