@@ -46,6 +46,7 @@ struct WideArgs {
   int H, G, T, S, DK, rep, causal;
   float scale_log2;
   int dv_half;  // value columns blockIdx.z * dv_half .. +dv_half of a wider head (0: one launch covers DV)
+  int by_tile;  // work order: tiles of all (batch, group, half) streams side by side (see wide_tile)
 };
 
 template <int DKP, int DV, int NBUF>
@@ -355,27 +356,41 @@ struct WideTile {
 // workgroup past the last slot tile (uniform over the workgroup).
 template <int SPT>
 __device__ __forceinline__ bool wide_tile(WideArgs& p, WideTile& t) {
-  // a head of 2 DV value columns in two halves (blockIdx.z): each half recomputes the same scores and softmax and
-  // accumulates its own columns, so both halves' outputs are those of one pass over all columns; half 0 writes LSE
-  if (p.dv_half) {
-    p.v += blockIdx.z * p.dv_half;
-    p.out += blockIdx.z * p.dv_half;
-    if (blockIdx.z) p.lse = nullptr;
-  }
   // XCD-aware order: workgroups are dealt round-robin over the 8 XCDs (flat id f runs on XCD f % 8); work item
   // w = bg * tiles + tile goes to XCD (w's range), so the slot tiles of one (batch, KV group) share an L2 for the
   // K/V they all stream. A bijection of [0, tiles * B G). Causal with the queries' own triangle at least half of
   // the keys (a prefill): a tile's work grows with its index, so each (batch, group) deals its tiles last first and
   // the light tiles fill the end instead of the heaviest ones (4 x 4096-token causal prefill, 32 / 8 heads of 128: 761 -> 703 us).
+  // by_tile (B G not a multiple of 8, where an XCD's range cuts a (batch, group) and gets its heavy or its light part):
+  // item f is tile f / streams of stream f % streams, a stream being a (batch, group, half); all streams deal their
+  // heaviest tiles first, and where the streams are a multiple of 8 each stays on one XCD (3 left-padded states of 1537
+  // tokens, 16 / 4 heads of 256, with the skipped blocks: 146 -> 95 us).
+  const bool last_first = p.causal && 2 * p.T >= p.S;
   const int tiles = gridDim.x, total = gridDim.x * gridDim.y;
-  const int f = blockIdx.x + blockIdx.y * tiles;
-  const int per = total >> 3, rem = total & 7, xcd = f & 7, local = f >> 3;
-  const int w = xcd < rem ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
-  const int bg = w / tiles;
+  int f = blockIdx.x + blockIdx.y * tiles, half = blockIdx.z, bg, tile;
+  if (p.by_tile) {
+    f += half * total;
+    const int groups = gridDim.y, streams = groups * gridDim.z, st = f % streams;
+    bg = st % groups;
+    half = st / groups;
+    tile = f / streams;
+  } else {
+    const int per = total >> 3, rem = total & 7, xcd = f & 7, local = f >> 3;
+    const int w = xcd < rem ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
+    bg = w / tiles;
+    tile = w % tiles;
+  }
+  if (last_first) tile = tiles - 1 - tile;
   t.b = bg / p.G;
   t.g = bg % p.G;
   const int nslots = p.T * p.rep;
-  const int tile = p.causal && 2 * p.T >= p.S ? tiles - 1 - w % tiles : w % tiles;
+  // a head of 2 DV value columns in two halves: each half recomputes the same scores and softmax and accumulates its
+  // own columns, so both halves' outputs are those of one pass over all columns; half 0 writes the LSE
+  if (p.dv_half) {
+    p.v += half * p.dv_half;
+    p.out += half * p.dv_half;
+    if (half) p.lse = nullptr;
+  }
   const int slot_base = tile * SPT;
   if (slot_base >= nslots) return false;
 
@@ -393,6 +408,31 @@ __device__ __forceinline__ bool wide_tile(WideArgs& p, WideTile& t) {
   t.nb = (kend + kBK - 1) / kBK;
   t.free_until = (slot_base + wave * 32) / p.rep + shift;
   return true;
+}
+
+// The first of the tile's nb blocks that holds a key kvalid keeps (nb: none): a left-padded state's leading blocks add
+// nothing, not even to the running max, and are not read. `first` is LDS; every thread of the workgroup takes part.
+__device__ __forceinline__ int first_block(const WideArgs& p, const WideTile& t, int& first) {
+  if (!p.kvalid) return 0;
+  const uint8_t* row = p.kvalid + (int64_t)t.b * p.smb;
+  const int tid = threadIdx.x, end = min(t.nb * kBK, p.S);
+  if (tid == 0) first = 0x7fffffff;
+  __syncthreads();
+  for (int j0 = 0; j0 < end; j0 += 4 * kThreads) {
+    int v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = j0 + i * kThreads + tid < end ? row[j0 + i * kThreads + tid] : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint64_t any = __builtin_amdgcn_ballot_w64(v[i] != 0);
+      if (any && (tid & 63) == 0) atomicMin(&first, j0 + i * kThreads + tid);  // the wave's 64 keys are one block
+    }
+    __syncthreads();
+    const int got = first;
+    __syncthreads();  // every thread has read it before a later round writes it
+    if (got != 0x7fffffff) return __builtin_amdgcn_readfirstlane(got / kBK);
+  }
+  return t.nb;
 }
 
 // query fragments: lane holds Q[slot][ks*16 + 8h .. +8], zero past DK
@@ -437,6 +477,7 @@ __device__ __forceinline__ void wide_epilogue(const WideArgs& p, const WideTile&
 template <int DKP, int DV, int NBUF, int OCC>
 __global__ __launch_bounds__(kThreads, OCC) void wide_attn_kernel(WideArgs p) {
   __shared__ WSmem<DKP, DV, NBUF> sm;
+  __shared__ int first;
   WideTile t;
   if (!wide_tile<kSlotsPerTile>(p, t)) return;
   const int lane = threadIdx.x & 63;
@@ -447,14 +488,14 @@ __global__ __launch_bounds__(kThreads, OCC) void wide_attn_kernel(WideArgs p) {
   v16f o[DV / 32];
 #pragma unroll
   for (int dt = 0; dt < DV / 32; ++dt) o[dt] = v16f{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const int nb = t.nb;
-  if (nb > 0) {
+  const int nb = t.nb, b0 = first_block(p, t, first);
+  if (b0 < nb) {
     BlockRegs<DKP, DV> br;
-    block_load<DKP, DV>(p, t.b, t.g, 0, br);
+    block_load<DKP, DV>(p, t.b, t.g, b0 * kBK, br);
     block_store<DKP, DV, NBUF>(sm, 0, br);
     __syncthreads();
-    for (int blk = 0; blk < nb; ++blk) {
-      const int cur = NBUF == 2 ? (blk & 1) : 0;
+    for (int blk = b0; blk < nb; ++blk) {
+      const int cur = NBUF == 2 ? ((blk - b0) & 1) : 0;
       const int j0 = blk * kBK;
       wide_block<DKP, DV, 1>(
           sm.k[cur], sm.kb[cur], sm.mk[cur],
@@ -533,6 +574,7 @@ __global__ __launch_bounds__(kThreads, OCC) void wide_dma_kernel(WideArgs p) {
   constexpr int KI = kBK * DKP * 2 / 4096;  // DMA rounds per block: a round moves 4 KB (16 bytes x 256 lanes)
   constexpr int VI = kBK * DV * 2 / 4096;
   __shared__ WDSmem<DKP> sm;
+  __shared__ int first;
   WideTile t;
   if (!wide_tile<kSlotsPerTile>(p, t)) return;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -597,13 +639,13 @@ __global__ __launch_bounds__(kThreads, OCC) void wide_dma_kernel(WideArgs p) {
     }
   };
 
-  const int nb = t.nb;
-  if (nb > 0) {
-    issue(0);
-    put_bias(key_ok(0));
+  const int nb = t.nb, b0 = first_block(p, t, first);
+  if (b0 < nb) {
+    issue(b0 * kBK);
+    put_bias(key_ok(b0 * kBK));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    for (int blk = 0; blk < nb; ++blk) {
+    for (int blk = b0; blk < nb; ++blk) {
       const int j0 = blk * kBK;
       const bool more = blk + 1 < nb;
       const int ok_next = more ? key_ok(j0 + kBK) : 0;
@@ -678,7 +720,8 @@ extern "C" int od_wide_attn(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t
   const int64_t tiles = (T * rep + kSlotsPerTile - 1) / kSlotsPerTile;
   if (tiles > 0x7fffffff || B * G > 65535 || T * rep > 0x7fffffff || S > 0x7fffffff - kBK) return OD_ERR_SHAPE;
   WideArgs a{q, k, v, kvalid, out, lse, sqb, sqh, sqt, skb, skg, sks, svb, svg, svs, sob, soh, sot, smb,
-             (int)H, (int)G, (int)T, (int)S, (int)DK, (int)rep, causal ? 1 : 0, scale * 1.4426950408889634f, 0};
+             (int)H, (int)G, (int)T, (int)S, (int)DK, (int)rep, causal ? 1 : 0, scale * 1.4426950408889634f, 0,
+             B * G % 8 != 0 && tiles * B * G <= 0x3fffffff ? 1 : 0};
   dim3 grid((unsigned)tiles, (unsigned)(B * G));
   hipStream_t st = (hipStream_t)stream;
   const int dkp = DK <= 64 ? 64 : DK <= 128 ? 128 : DK <= 256 ? 256 : 512;

@@ -156,3 +156,23 @@ def test_scale_must_be_positive():
     for bad in (0.0, -0.125):
         with pytest.raises(ValueError):
             wide_attention(q.to(DEV), k.to(DEV), v.to(DEV), bad)
+
+
+@pytest.mark.parametrize("B,H,G,T,S,DK,DV,pads,causal", [
+    (3, 4, 1, 200, 200, 128, 128, [0, 64, 190], True), (3, 8, 2, 130, 1300, 128, 128, [1100, 1024, 1299], True),
+    (3, 4, 2, 150, 150, 256, 256, [63, 65, 150], True), (5, 2, 1, 70, 300, 64, 128, [0, 300, 128, 127, 1], False),
+    (3, 4, 1, 90, 200, 200, 128, [130, 0, 64], True), (2, 6, 3, 260, 260, 64, 64, [100, 256], True)])
+def test_left_pads_and_stream_order(gpu_lib, B, H, G, T, S, DK, DV, pads, causal):
+    """Left-padded states, whose leading blocks are skipped: pads of no, whole and partial 64-key blocks, past the first
+    1024 keys scanned, over every key (outputs 0, LSE -inf) and over every key that early queries see; on the LDS-DMA
+    path with and without halves and on the register-staged path; (batch, group) counts that are not multiples of 8
+    (tiles of all streams side by side), with 1 and 2 halves."""
+    q, k, v, _ = make(B * 100 + S + DK, B, H, G, T, S, DK, DV, False)
+    kv = torch.arange(S)[None, :] >= torch.tensor(pads)[:, None]
+    out, lse = run(q, k, v, kv, causal)
+    ob, lb, bound = oa.wide_attention_blocked(q, k, v, DK ** -0.5, kv, causal, with_bound=True)
+    check_vs_blocked(out.cpu().float(), ob, bound, f"left pads {pads}")
+    ref = oa.attention(q, k, v, DK ** -0.5, kv, causal, dtype=torch.float64)[1].float()
+    got = lse.cpu()
+    assert torch.equal(got.isinf(), ref.isinf())
+    assert (got - ref)[~ref.isinf()].abs().max().item() <= 1e-4 if (~ref.isinf()).any() else True
