@@ -361,10 +361,8 @@ __device__ __forceinline__ bool wide_tile(WideArgs& p, WideTile& t) {
   // K/V they all stream. A bijection of [0, tiles * B G). Causal with the queries' own triangle at least half of
   // the keys (a prefill): a tile's work grows with its index, so each (batch, group) deals its tiles last first and
   // the light tiles fill the end instead of the heaviest ones (4 x 4096-token causal prefill, 32 / 8 heads of 128: 761 -> 703 us).
-  // by_tile (B G not a multiple of 8, where an XCD's range cuts a (batch, group) and gets its heavy or its light part):
-  // item f is tile f / streams of stream f % streams, a stream being a (batch, group, half); all streams deal their
-  // heaviest tiles first, and where the streams are a multiple of 8 each stays on one XCD (3 left-padded states of 1537
-  // tokens, 16 / 4 heads of 256, with the skipped blocks: 146 -> 95 us).
+  // by_tile: item f is tile f / streams of stream f % streams, a stream being a (batch, group, half). All streams deal
+  // their heaviest tiles first, so no XCD ends with the heavy tiles of the stream that its range ends in.
   const bool last_first = p.causal && 2 * p.T >= p.S;
   const int tiles = gridDim.x, total = gridDim.x * gridDim.y;
   int f = blockIdx.x + blockIdx.y * tiles, half = blockIdx.z, bg, tile;
@@ -720,8 +718,16 @@ extern "C" int od_wide_attn(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t
   const int64_t tiles = (T * rep + kSlotsPerTile - 1) / kSlotsPerTile;
   if (tiles > 0x7fffffff || B * G > 65535 || T * rep > 0x7fffffff || S > 0x7fffffff - kBK) return OD_ERR_SHAPE;
   WideArgs a{q, k, v, kvalid, out, lse, sqb, sqh, sqt, skb, skg, sks, svb, svg, svs, sob, soh, sot, smb,
-             (int)H, (int)G, (int)T, (int)S, (int)DK, (int)rep, causal ? 1 : 0, scale * 1.4426950408889634f, 0,
-             B * G % 8 != 0 && tiles * B * G <= 0x3fffffff ? 1 : 0};
+             (int)H, (int)G, (int)T, (int)S, (int)DK, (int)rep, causal ? 1 : 0, scale * 1.4426950408889634f, 0, 0};
+  // The tiles of all streams side by side (wide_tile) where a tile's work varies, causal over at most four times the
+  // queries' keys: with an XCD's contiguous range cutting a (batch, group) (B G not a multiple of 8) at every size (3
+  // left-padded states of 1537 tokens, 16 / 4 heads of 256, with the skipped blocks 146 -> 95 us; 1 x 32768 of the same
+  // heads 8.8 -> 5.9 ms), else with up to 96 MB of K and V (8 x 2048 tokens, 32 / 8 heads of 128: 191 -> 174 us;
+  // 2 x 1000: 43 -> 37). Above it an XCD reads all its streams' K/V at once and misses the caches (8 x 4000 tokens
+  // after 3900, 32 / 8 heads: 1613 us in ranges, 1736 side by side), as over more keys, where the tiles are alike
+  // (3 x 1000 tokens after 8000, 12 / 4 heads: 141 and 146 us).
+  a.by_tile = causal && 4 * T >= S && (B * G % 8 != 0 || B * G * S * (DK + DV) <= (48 << 20)) &&
+              tiles * B * G <= 0x3fffffff;
   dim3 grid((unsigned)tiles, (unsigned)(B * G));
   hipStream_t st = (hipStream_t)stream;
   const int dkp = DK <= 64 ? 64 : DK <= 128 ? 128 : DK <= 256 ? 256 : 512;
