@@ -276,6 +276,56 @@ def test_gdn_one_chunk_rows(gpu_lib, S, L, n_k, n_v, dv, states):
     assert (d.norm() / o_r.norm()).item() <= 2e-3
 
 
+@pytest.mark.parametrize("S,L,n_k,n_v", [(1, 1, 1, 1), (2, 15, 1, 2), (1, 16, 2, 6), (1, 17, 2, 4), (3, 31, 1, 3),
+                                         (1, 32, 2, 4), (2, 33, 2, 2), (2, 48, 1, 2)])
+@pytest.mark.parametrize("same_key", [False, True])
+def test_gdn_chunk_t_matches_float64(gpu_lib, S, L, n_k, n_v, same_key):
+    """T = (I + A)^{-1} diag(beta), as the chunk workspace holds it (bf16 hi + lo), against a float64 triangular solve:
+    chunks that end in either 16-token block, one to three value heads per key head, and one key for all tokens with
+    beta = 0.999. Bound: the split's 2^-16 |T|, 32u |X| |I + A| |T| of a forward substitution (u = 2^-24, X = (I + A)^{-1};
+    the factor 4 covers the block form's three products), and |X| dA |T| with dA from the 128-term product of
+    the keys, the 32-term sum of the gates and the exponential (4 ulp and 2u per unit of its argument)."""
+    from opendecider_amd import kernels
+    from opendecider_amd._lib import check, lib, ptr, stream_of
+    g = torch.Generator().manual_seed(S * 1000 + L + n_v)
+    q, k, v, gg, beta = _rec_inputs(g, S, L, n_k, n_v)
+    if same_key:
+        k = k.reshape(S * L, n_k, 128)[:1].expand(S * L, -1, -1).reshape(k.shape).contiguous()
+        beta = torch.full_like(beta, 0.999)
+        gg = gg * 0.01
+    print(f"gdn T S={S} L={L} n_k={n_k} n_v={n_v} same_key={same_key}", flush=True)
+    qk = torch.cat([q.reshape(S * L, -1), k.reshape(S * L, -1)], 1).to(DEV)
+    o = torch.empty(S * L, n_v * 128, dtype=torch.bfloat16, device=DEV)
+    ws = torch.zeros(kernels.gdn_chunk_workspace_floats(S, L, n_v), device=DEV)
+    vd, gd, bd = v.reshape(S * L, -1).to(DEV), gg.to(DEV), beta.to(DEV)
+    check(lib().od_gdn_recurrence_chunked(ptr(qk), ptr(vd), ptr(gd), ptr(bd), ptr(None), ptr(None), 0, S, L, n_k, n_v,
+                                          128, 128, ptr(o), ptr(None), ptr(ws), ws.numel(), stream_of(qk)),
+          "od_gdn_recurrence_chunked")
+    nc, rep = (L + 31) // 32, n_v // n_k
+    hl = ws.cpu()[:S * nc * n_v * 1136].reshape(S, nc, n_v, 1136)[..., :1024].contiguous().view(torch.bfloat16)
+    hl = hl.reshape(S, nc, n_v, 2, 32, 32).double()
+
+    def chunks(x, heads):  # [S L, heads, ...] -> [S, nc, heads, 32, ...]
+        x = x.reshape(S, L, heads, -1).double()
+        return torch.nn.functional.pad(x, (0, 0, 0, 0, 0, nc * 32 - L)).reshape(S, nc, 32, heads, -1).transpose(2, 3)
+    kc = chunks(k, n_k).repeat_interleave(rep, 2)
+    gc, bc = chunks(gg, n_v)[..., 0], chunks(beta, n_v)[..., 0]
+    gam = gc.cumsum(-1)
+    e = bc[..., :, None] * torch.exp(gam[..., :, None] - gam[..., None, :]).tril(-1)
+    kk = kc @ kc.transpose(-1, -2)
+    eye = torch.eye(32, dtype=torch.float64)
+    IA = eye + (e * kk).tril(-1)
+    T = torch.linalg.solve_triangular(IA, torch.diag_embed(bc), upper=False)
+    X = torch.linalg.solve_triangular(IA, eye.expand_as(IA), upper=False)
+    u = 2.0 ** -24
+    n2 = kc.norm(dim=-1)
+    span = gc.abs().sum(-1)[..., None, None]
+    dA = e * (128 * u * n2[..., :, None] * n2[..., None, :] + kk.abs() * u * (10 + 66 * span))
+    bound = 2.0 ** -16 * T.abs() + 4 * 32 * u * X.abs() @ IA.abs() @ T.abs() + X.abs() @ dA @ T.abs()
+    err = (hl[..., 0, :, :] + hl[..., 1, :, :] - T).abs()
+    assert (err <= bound + 1e-30).all(), (err - bound).max().item()
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 def test_gdn_recurrence_in_place_state_and_continuation(gpu_lib, chunked):
     """Running L1 tokens, then L2 more continuing the written state in place, equals one run over L1 + L2 tokens up
