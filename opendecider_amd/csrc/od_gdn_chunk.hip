@@ -14,7 +14,7 @@
 // gdn_chunk_t, per (sequence, chunk, key head): K K^T on MFMA and T in fp32, by forward substitution in two blocks,
 // for each value head of that key head, written as bf16 hi / lo in the layout the second kernel copies straight into
 // LDS, with the vectors gamma, e^gamma, e^{gamma_C - gamma} and e^{gamma_C}. Then, chunk after chunk (the only
-// sequential part), gdn_chunk_roles (two or more chunks; a role per wave) or gdn_chunk_state (one chunk), both per
+// sequential part), gdn_chunk_roles (a role per wave) or gdn_chunk_state (one chunk, see the dispatch), both per
 // (sequence, value head, 64 state columns) with 16 columns per wave; gdn_chunk_state takes P from
 // K Q~^T on MFMA, then the products above. The state lives in the MFMA accumulators
 // (V_MFMA_F32_16X16X32_BF16, lane l: column l % 16, rows 4 (l / 16) + i of each 16 x 16 tile) and feeds the next
@@ -899,7 +899,10 @@ extern "C" int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, 
   TArgs tp{qk, g, beta, ws, L, nchunk, (int)n_k, (int)n_v};
   gdn_chunk_t_kernel<<<dim3((unsigned)tblocks), dim3(64), 0, (hipStream_t)stream>>>(tp);
   CArgs cp{qk, v, init, seq_state, ws, o, final_state, L, nchunk, n_states, (int)n_k, (int)n_v, (int)dv, S, 1};
-  // One chunk and no state kept (option rows): runs of sequences that share S_0 in registers, a workgroup per CU.
+  // One chunk and no state kept (option rows): runs of sequences that share S_0 in registers, a workgroup per CU (256 x
+  // 24 tokens over 4 states, 32 heads, with T: 227 us on gdn_chunk_state, 75 here; 6 x 24: 17.4 and 12.8). Its eight
+  // chain waves take 128 columns; other widths, and a state that has to be written per sequence (2 MB each, which is
+  // what such a call then takes its time for), stay on gdn_chunk_state.
   if (nchunk == 1 && !final_state && dv % (16 * kRowChain) == 0) {
     const int64_t heads = n_v * (dv / (16 * kRowChain));
     cp.run = (int)min((int64_t)kMaxRun, max((int64_t)1, S * heads / 256));
@@ -907,7 +910,7 @@ extern "C" int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, 
     gdn_chunk_roles_kernel<true><<<dim3((unsigned)blocks), dim3(64 * (kRowChain + 4)), 0, (hipStream_t)stream>>>(cp);
     return od_launch_status();
   }
-  // Two or more chunks: a role per wave (4 x 4096 tokens, 32 heads, both kernels: 508 -> 231 us; 1 x 8192: 887 -> 322;
+  // Two or more chunks: a role per wave (4 x 4096 tokens, 32 heads, both kernels: 508 -> 220 us; 1 x 8192: 887 -> 322;
   // 2 chunks of 64 sequences: 115 -> 112). Its one workgroup per CU loses to three of the other where two chunks come
   // with more work than about 16 workgroups per CU (2 chunks of 256 sequences: 385 -> 401).
   if (nchunk > 2 || (nchunk == 2 && cblocks <= 4096))
