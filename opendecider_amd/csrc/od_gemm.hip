@@ -680,7 +680,7 @@ __global__ __launch_bounds__(kThreads, BM == 128 && BN == 128 && NS == 2 ? 4 : 1
 // The small-M kernel (M up to a few hundred rows and few tiles: a single 256-row linear, the question and record
 // passes): the 256-row tiles above leave most CUs idle there, and splitting K across workgroups costs int32 partial
 // planes in memory (2 x splits x M x N x 4 bytes) and a second launch. Here one workgroup of 4 waves owns a
-// 64 x BN tile and splits K inside itself: wave w sums the 128-byte k-chunks w, w + 4, w + 8, ... of the tile. Each
+// 64 x BN tile (small_bn) and splits K inside itself: wave w sums the 128-byte k-chunks w, w + 4, w + 8, ... of the tile. Each
 // wave has two LDS buffers of its own (a chunk's 64 A rows and BN W rows, 128 bytes each, in the swizzled layout of
 // the 256-row kernel) and moves its next chunk in by LDS DMA (8 lanes per 128-byte line; rows past M / N and bytes
 // past K read as zeros) while it computes the current one, so the waves never wait for each other until the end.
@@ -893,15 +893,27 @@ struct SplitPlan {
 
 // Shapes for the small-M kernel (w8a8_gemm_small_kernel): up to 512 rows and at most two of its 64 x 64 tiles per
 // CU (it runs one workgroup per CU and pays each tile's first-chunk latency in full; M = 512 x N = 6144 is faster on
-// the 128 x 256 tiles with split-K). Its tile width: 64 columns when that gives every CU a tile, else 32 (twice the
-// tiles, each reading A again).
+// the 128 x 256 tiles with split-K). Its tile width, 32, 64 or 96 columns: the one whose rounds of one tile per CU
+// take the least. The 64 rows of A are read whatever the width: one round at K = 4096 measures 8.0, 12.0 and 16.7 us
+// (10.4, 13.9 and 18.5 with W from HBM), 0.67 and 1.33 of the 64-wide one. 192 x 4096 x 12288 in one round of 64 takes
+// 31 us, in two of 32 42; 256 x 6144 x 4096 in one round of 96 18.5, in two of 64 26.
 constexpr int64_t kSmallMaxM = 512;
 bool small_m(int64_t M, int64_t N) {
   return M <= kSmallMaxM && ((M + kSmBM - 1) / kSmBM) * ((N + 63) / 64) <= 2 * (int64_t)cu_count();
 }
 int small_bn(int64_t M, int64_t N) {
-  const int64_t tiles64 = ((M + kSmBM - 1) / kSmBM) * ((N + 63) / 64);
-  return tiles64 >= cu_count() ? 64 : 32;
+  const int64_t tm = (M + kSmBM - 1) / kSmBM, cus = cu_count();
+  int best = 64;
+  double t = 1e30;
+  for (const int bn : {64, 32, 96}) {
+    const int64_t rounds = (tm * ((N + bn - 1) / bn) + cus - 1) / cus;
+    const double e = (double)rounds * (bn == 32 ? 0.67 : bn == 64 ? 1.0 : 1.33);
+    if (e < t) {
+      t = e;
+      best = bn;
+    }
+  }
+  return best;
 }
 
 SplitPlan split_plan(int64_t M, int64_t N, int64_t K) {
@@ -985,7 +997,10 @@ int gemm_launch(const GemmArgs& p0, bool swiglu, hipStream_t st, const SplitPlan
     p.tiles_m = (int)tiles_m;
     p.tiles_n = (int)tiles_n;
     const dim3 grid((unsigned)(tiles_m * tiles_n)), block(kSmWaves * 64);
-    if (bn == 64) {
+    if (bn == 96) {
+      swiglu ? w8a8_gemm_small_kernel<96, true><<<grid, block, 0, st>>>(p)
+             : w8a8_gemm_small_kernel<96, false><<<grid, block, 0, st>>>(p);
+    } else if (bn == 64) {
       swiglu ? w8a8_gemm_small_kernel<64, true><<<grid, block, 0, st>>>(p)
              : w8a8_gemm_small_kernel<64, false><<<grid, block, 0, st>>>(p);
     } else {

@@ -484,6 +484,28 @@ def test_small_m_kernel_bit_identical_to_256_row_kernel(gpu_lib, M, N, K, epi):
         assert torch.equal(got.cpu(), refo)
 
 
+@pytest.mark.parametrize("M,N,K,epi", [(3, 24570, 48, "plain"), (200, 5199, 272, "bias"), (256, 6144, 128, "res"),
+                                       (512, 2101, 144, "bias_res"), (33, 20482, 160, "swiglu"), (250, 6142, 400, "swiglu"),
+                                       (129, 4096, 1040, "res"), (192, 5456, 1168, "bias"), (150, 4102, 272, "swiglu")])
+def test_small_m_tile_widths(gpu_lib, M, N, K, epi):
+    """The small-M kernel's 96-column tiles (more than one round of 64-column ones) and its 64-column tiles where two
+    rounds of 32 would be needed, with ragged M, N and K tails: the oracle's bits."""
+    from opendecider_amd import kernels
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w, sa, sw = _gemm_case(g, M, N, K)
+    bias = torch.randn(N, generator=g).to(torch.bfloat16) if "bias" in epi else None
+    res = torch.randn(M, N, generator=g).to(torch.bfloat16) if "res" in epi else None
+    print(f"small-M widths M={M} N={N} K={K} {epi}", flush=True)
+    ref = oq.w8a8_epilogue(oq.int_gemm(a, w), sa, sw, bias, res)
+    if epi == "swiglu":
+        got = kernels.w8a8_gemm_swiglu(a.to(DEV), sa.to(DEV), w.to(DEV), sw.to(DEV))
+        ref = od.swiglu(ref[:, torch.cat([torch.arange(0, N, 2), torch.arange(1, N, 2)])], N // 2)
+    else:
+        got = kernels.w8a8_gemm(a.to(DEV), sa.to(DEV), w.to(DEV), sw.to(DEV), None if bias is None else bias.to(DEV),
+                                None if res is None else res.to(DEV))
+    assert torch.equal(got.cpu(), ref.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(1024, 2048, 6144, "plain"), (600, 1030, 6144, "swiglu"),
                                        (1024, 4096, 12288, "res"), (700, 2048, 6144, "bias_res"),
                                        (1000, 20, 2064, "bias_res")])
