@@ -528,9 +528,10 @@ __global__ __launch_bounds__(256) void gdn_chunk_state_kernel(CArgs p) {
 // against 6500 with every wave doing all of it, 476 -> 175 us; one workgroup per CU, LDS 110 KB).
 // Rows of K, Q, V, T and P are staged in the order row(j) = 16 ((j >> 2) & 1) + 4 (j >> 3) + (j & 3) and the state's dk
 // rows alike within each 32, which makes accumulator tiles 0 and 1 of a lane group h hold tokens (dk) 8 h .. 8 h + 7 in
-// order: every operand is then one 16-byte LDS read in natural order, K^T and V^T two transposing reads. Y and O are taken transposed (the state as the A
-// operand), so a lane holds four neighbouring columns of a token and the outputs leave as 8-byte LDS writes.
-// row strides of 32 bytes past a multiple of 64: a fragment read (row lane % 16, 16 bytes at lane / 16) is then free
+// order: every operand is then one 16-byte LDS read in natural order, K^T and V^T two transposing reads. Y and O are
+// taken transposed (the state as the A operand), so a lane holds four neighbouring columns of a token and the outputs
+// leave as 8-byte LDS writes.
+// Row strides of 32 bytes past a multiple of 64: a fragment read (row lane % 16, 16 bytes at lane / 16) is then free
 // of bank conflicts (ds_read_b128 serves lanes 0-3, 12-15, 20-27 together, and so on: strides of 80 and 272 bytes
 // took two cycles for one, measured)
 constexpr int kRowK2 = kDk + 16;

@@ -680,7 +680,7 @@ __global__ __launch_bounds__(kThreads, BM == 128 && BN == 128 && NS == 2 ? 4 : 1
 // The small-M kernel (M up to a few hundred rows and few tiles: a single 256-row linear, the question and record
 // passes): the 256-row tiles above leave most CUs idle there, and splitting K across workgroups costs int32 partial
 // planes in memory (2 x splits x M x N x 4 bytes) and a second launch. Here one workgroup of 4 waves owns a
-// 64 x BN tile (small_bn) and splits K inside itself: wave w sums the 128-byte k-chunks w, w + 4, w + 8, ... of the tile. Each
+// 64 x BN tile (small_bn) and splits K inside itself: wave w sums the tile's 128-byte k-chunks w, w + 4, w + 8, ... Each
 // wave has two LDS buffers of its own (a chunk's 64 A rows and BN W rows, 128 bytes each, in the swizzled layout of
 // the 256-row kernel) and moves its next chunk in by LDS DMA (8 lanes per 128-byte line; rows past M / N and bytes
 // past K read as zeros) while it computes the current one, so the waves never wait for each other until the end.

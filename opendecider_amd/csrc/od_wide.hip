@@ -360,7 +360,8 @@ __device__ __forceinline__ bool wide_tile(WideArgs& p, WideTile& t) {
   // w = bg * tiles + tile goes to XCD (w's range), so the slot tiles of one (batch, KV group) share an L2 for the
   // K/V they all stream. A bijection of [0, tiles * B G). Causal with the queries' own triangle at least half of
   // the keys (a prefill): a tile's work grows with its index, so each (batch, group) deals its tiles last first and
-  // the light tiles fill the end instead of the heaviest ones (4 x 4096-token causal prefill, 32 / 8 heads of 128: 761 -> 703 us).
+  // the light tiles fill the end instead of the heaviest ones (4 x 4096-token causal prefill, 32 / 8 heads of 128: 761
+  // -> 703 us).
   // by_tile: item f is tile f / streams of stream f % streams, a stream being a (batch, group, half). All streams deal
   // their heaviest tiles first, so no XCD ends with the heavy tiles of the stream that its range ends in.
   const bool last_first = p.causal && 2 * p.T >= p.S;
