@@ -559,13 +559,14 @@ int od_w8a8_linear(const uint16_t* x, int64_t ldx, const uint16_t* inv_s, const 
  * Decision readout of the option rows (src/opendecider/v3.py:639-643,701-709, src/opendecider/decider.py:255-257):
  *   h bf16 [B n_opt t, H] (row stride ldh), final_norm bf16 [H], head fp32 [H], none_logit fp32 [1]. Per token the final
  *   RMSNorm hn = bf16(w * bf16(h * r)) (norm_offset: bf16((h * r) * (1 + w))), r as od_rmsnorm_quant takes it; per
- *   option row the mean over its tokens t0 .. t - 1 of hn . head (float64 sums, rounded once) into logits fp32
- *   [B n_opt] (a workspace of the caller); per request log_softmax([logits ; none_logit] * inv_temperature) into out
- *   fp32 [B, n_opt + 1]. 0 <= t0 < t. Two launches.
+ *   option row its logit, the mean over its tokens t0 .. t - 1 of hn . head (float64 sums, rounded once to fp32); per
+ *   request log_softmax([logits ; none_logit] * inv_temperature) into out fp32 [B, n_opt + 1]. 0 <= t0 < t. A row's
+ *   tokens are summed by `chunks` workgroups (at least 1; no more than t - t0 are used) into part, a workspace of the
+ *   caller of B n_opt chunks float64. Two launches.
  */
 int od_readout(const uint16_t* h, int64_t ldh, const uint16_t* final_norm, int norm_offset, float eps,
                const float* head, const float* none_logit, float inv_temperature, int64_t B, int64_t n_opt, int64_t t,
-               int64_t t0, int64_t H, float* logits, float* out, od_stream_t stream);
+               int64_t t0, int64_t H, int64_t chunks, double* part, float* out, od_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -90,7 +90,7 @@ SIGNATURES = {
     "od_w8a8_linear": [_c_ptr, _i64, _c_ptr, _c_ptr, _i64, _c_ptr, _c_ptr, _c_ptr, _i64, _c_ptr, _i64, _c_ptr, _c_ptr,
                        _i64, _i64, _i64, _c_ptr, _i64, _c_ptr],
     "od_readout": [_c_ptr, _i64, _c_ptr, ctypes.c_int, ctypes.c_float, _c_ptr, _c_ptr, ctypes.c_float, _i64, _i64, _i64,
-                   _i64, _i64, _c_ptr, _c_ptr, _c_ptr],
+                   _i64, _i64, _i64, _c_ptr, _c_ptr, _c_ptr],
     "od_lm_head_logprob_ws": [_i64, _i64, _c_ptr],
     "od_lm_head_logprob": [_c_ptr, _i64, _c_ptr, _i64, ctypes.c_int, _c_ptr, _i64, _c_ptr, _c_ptr, _i64, _i64, _i64,
                            _c_ptr, _c_ptr, _i64, _c_ptr],

@@ -479,25 +479,29 @@ struct ReadoutArgs {
   const uint16_t* w;
   const float* head;
   const float* none;
-  float* logits;
+  double* part;
   float* out;
   int64_t ldh, H;
   int n_opt, t, t0, vec;
+  int chunks, per;  // workgroups of an option row, tokens of each
   float eps, inv_temp;
 };
 
-// One workgroup per option row, its tokens shared out over the waves; a token's values are read twice (the sum of
-// squares, then the normed dot product: the second read hits the cache). Bound by the latency of those reads: one
-// launch over 32 MB in place of a dozen elementwise ones over float32 and float64 copies of it (4096 tokens x 4096:
-// about 250 -> 16 us).
+// p.chunks workgroups per option row, the tokens of a chunk shared out over the waves; a token's values are read twice
+// (the sum of squares, then the normed dot product: the second read hits the cache). Bound by the latency of those
+// reads, 4 to 5 us for a wave's token of 4096 values, so a row is cut up while the chip has room (readout_chunks): a
+// whole call of one row of 4096 tokens took 5465 us on one workgroup (271 with torch operators) and takes 19 cut up,
+// 2 rows of 256 248 (96) and 13.6, 256 rows of 16 24 (264) and 15.4.
 constexpr int kReadoutThreads = 256;
 template <bool OFFSET>
 __global__ __launch_bounds__(kReadoutThreads) void readout_rows_kernel(ReadoutArgs p) {
   __shared__ double red[kReadoutThreads / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double dot = 0.0;
-  for (int j = p.t0 + wave; j < p.t; j += kReadoutThreads / 64) {
-    const uint16_t* row = p.h + ((int64_t)blockIdx.x * p.t + j) * p.ldh;
+  const int64_t opt = blockIdx.x / p.chunks, lo = p.t0 + (int64_t)(blockIdx.x % p.chunks) * p.per;
+  const int64_t hi = min(lo + p.per, (int64_t)p.t);
+  for (int64_t j = lo + wave; j < hi; j += kReadoutThreads / 64) {
+    const uint16_t* row = p.h + (opt * p.t + j) * p.ldh;
     double ss = 0.0;
     const int64_t nv = p.vec ? p.H / 8 : 0;
     for (int64_t c = lane; c < nv; c += 64) {
@@ -543,16 +547,27 @@ __global__ __launch_bounds__(kReadoutThreads) void readout_rows_kernel(ReadoutAr
     double s = 0.0;
 #pragma unroll
     for (int i = 0; i < kReadoutThreads / 64; ++i) s += red[i];
-    p.logits[blockIdx.x] = (float)(s / (double)(p.t - p.t0));
+    p.part[blockIdx.x] = s;
   }
 }
 
-// log_softmax over a request's option logits and the none logit, one workgroup per request
+// The logits from their chunks' sums (G lanes per option, as many as the workgroup has for its options, up to 64), then
+// log_softmax over them and the none logit: one workgroup per request. `out` holds the scaled logits in between.
 __global__ __launch_bounds__(kReadoutThreads) void readout_softmax_kernel(ReadoutArgs p) {
   __shared__ float red[kReadoutThreads / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = p.n_opt + 1;
-  const float* x = p.logits + (int64_t)blockIdx.x * p.n_opt;
-  auto value = [&](int i) { return (i < p.n_opt ? x[i] : p.none[0]) * p.inv_temp; };
+  float* x = p.out + (int64_t)blockIdx.x * n;
+  int G = 64;
+  while (G > 1 && (G >= 2 * p.chunks || (int64_t)G * p.n_opt > kReadoutThreads)) G /= 2;
+  for (int i = threadIdx.x / G; i < p.n_opt; i += kReadoutThreads / G) {
+    const double* part = p.part + ((int64_t)blockIdx.x * p.n_opt + i) * p.chunks;
+    double s = 0.0;
+    for (int c = threadIdx.x % G; c < p.chunks; c += G) s += part[c];
+    for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, OD_WAVE);
+    if (threadIdx.x % G == 0) x[i] = (float)(s / (double)(p.t - p.t0)) * p.inv_temp;
+  }
+  if (threadIdx.x == 0) x[p.n_opt] = p.none[0] * p.inv_temp;
+  __syncthreads();
   auto reduce = [&](float v, bool mx) {
     for (int o = 32; o > 0; o >>= 1) {
       const float y = __shfl_xor(v, o, OD_WAVE);
@@ -566,12 +581,12 @@ __global__ __launch_bounds__(kReadoutThreads) void readout_softmax_kernel(Readou
     return v;
   };
   float m = -INFINITY;
-  for (int i = threadIdx.x; i < n; i += kReadoutThreads) m = fmaxf(m, value(i));  // (a NaN comes back through the sum)
+  for (int i = threadIdx.x; i < n; i += kReadoutThreads) m = fmaxf(m, x[i]);  // (a NaN comes back through the sum)
   m = reduce(m, true);
   float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += kReadoutThreads) s += expf(value(i) - m);
+  for (int i = threadIdx.x; i < n; i += kReadoutThreads) s += expf(x[i] - m);
   const float lse = logf(reduce(s, false));
-  for (int i = threadIdx.x; i < n; i += kReadoutThreads) p.out[(int64_t)blockIdx.x * n + i] = value(i) - m - lse;
+  for (int i = threadIdx.x; i < n; i += kReadoutThreads) x[i] = x[i] - m - lse;
 }
 
 
@@ -775,21 +790,24 @@ extern "C" int od_qk_norm_rope_kv_append(uint16_t* qkv, int64_t ld, int64_t B, i
 
 extern "C" int od_readout(const uint16_t* h, int64_t ldh, const uint16_t* final_norm, int norm_offset, float eps,
                           const float* head, const float* none_logit, float inv_temperature, int64_t B, int64_t n_opt,
-                          int64_t t, int64_t t0, int64_t H, float* logits, float* out, od_stream_t stream) {
-  if (B < 0 || n_opt < 0 || H < 1 || t < 1 || t0 < 0 || t0 >= t || ldh < H) return OD_ERR_SHAPE;
+                          int64_t t, int64_t t0, int64_t H, int64_t chunks, double* part, float* out,
+                          od_stream_t stream) {
+  if (B < 0 || n_opt < 0 || H < 1 || t < 1 || t0 < 0 || t0 >= t || ldh < H || chunks < 1) return OD_ERR_SHAPE;
   if (B == 0) return OD_OK;
   if (!none_logit || !out) return OD_ERR_NULL;
-  if (n_opt > 0 && (!h || !final_norm || !head || !logits)) return OD_ERR_NULL;
-  if (B * n_opt > 0x7fffffffll || B > 0x7fffffffll || n_opt >= 0x7fffffffll || t > 0x7fffffffll) return OD_ERR_SHAPE;
-  ReadoutArgs p{h, final_norm, head, none_logit, logits, out, ldh, H, (int)n_opt, (int)t, (int)t0,
-                ldh % 8 == 0 && od_aligned16(h) && od_aligned16(final_norm) && od_aligned16(head) ? 1 : 0, eps,
-                inv_temperature};
+  if (n_opt > 0 && (!h || !final_norm || !head || !part)) return OD_ERR_NULL;
+  if (chunks > t - t0) chunks = t - t0;
+  if (t > 0x7fffffffll || n_opt >= 0x7fffffffll || B > 0x7fffffffll || B * n_opt > 0x7fffffffll / chunks)
+    return OD_ERR_SHAPE;
+  ReadoutArgs p{h, final_norm, head, none_logit, part, out, ldh, H, (int)n_opt, (int)t, (int)t0,
+                ldh % 8 == 0 && od_aligned16(h) && od_aligned16(final_norm) && od_aligned16(head) ? 1 : 0,
+                (int)chunks, (int)((t - t0 + chunks - 1) / chunks), eps, inv_temperature};
   hipStream_t st = (hipStream_t)stream;
   if (n_opt > 0) {
     if (norm_offset)
-      readout_rows_kernel<true><<<dim3((unsigned)(B * n_opt)), dim3(kReadoutThreads), 0, st>>>(p);
+      readout_rows_kernel<true><<<dim3((unsigned)(B * n_opt * chunks)), dim3(kReadoutThreads), 0, st>>>(p);
     else
-      readout_rows_kernel<false><<<dim3((unsigned)(B * n_opt)), dim3(kReadoutThreads), 0, st>>>(p);
+      readout_rows_kernel<false><<<dim3((unsigned)(B * n_opt * chunks)), dim3(kReadoutThreads), 0, st>>>(p);
   }
   readout_softmax_kernel<<<dim3((unsigned)B), dim3(kReadoutThreads), 0, st>>>(p);
   return od_launch_status();

@@ -757,6 +757,12 @@ def wide_attn(q, k, v, scale: float, kvalid=None, causal: bool = True, return_ls
     return (out, lse) if return_lse else out
 
 
+def readout_chunks(rows: int, tokens: int, n_cu: int = 256) -> int:
+    """Workgroups that share an option row's tokens in od_readout: four tokens each (one per wave), but no more than
+    eight workgroups per CU over all rows (what a CU holds at once; more only queue, each with its own reduction)."""
+    return max(1, min(-(-tokens // 4), 8 * n_cu // max(rows, 1)))
+
+
 def readout(h: torch.Tensor, final_norm: torch.Tensor, head: torch.Tensor, none_logit: torch.Tensor, eps: float,
             temperature: float, B: int, n_opt: int, t: int, t0: int = 0, offset: bool = False) -> torch.Tensor:
     """od_readout: h (B n_opt t, H) bf16 with contiguous rows, final_norm (H,) bf16, head (H,) fp32, none_logit () fp32.
@@ -769,11 +775,12 @@ def readout(h: torch.Tensor, final_norm: torch.Tensor, head: torch.Tensor, none_
         raise ValueError("readout: h must be (B n_opt t, H) with contiguous rows")
     final_norm = _vec(final_norm, H, "final_norm")
     head, none_logit = _scales(head, H, "head"), _scales(none_logit, 1, "none_logit")
-    logits = torch.empty(max(B * n_opt, 1), dtype=torch.float32, device=h.device)
+    chunks = readout_chunks(B * n_opt, t - t0, cu_count(h.device))
+    part = torch.empty(max(B * n_opt * chunks, 1), dtype=torch.float64, device=h.device)
     out = torch.empty(B, n_opt + 1, dtype=torch.float32, device=h.device)
     check(lib().od_readout(ptr(h), h.stride(0) if h.shape[0] > 1 else H, ptr(final_norm), int(bool(offset)), float(eps),
-                           ptr(head), ptr(none_logit), 1.0 / float(temperature), B, n_opt, t, t0, H, ptr(logits),
-                           ptr(out), stream_of(h)), "od_readout")
+                           ptr(head), ptr(none_logit), 1.0 / float(temperature), B, n_opt, t, t0, H, chunks,
+                           ptr(part), ptr(out), stream_of(h)), "od_readout")
     return out
 
 

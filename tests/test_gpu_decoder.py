@@ -327,6 +327,23 @@ def test_readout_kernel(gpu_lib, B, n_opt, t, t0, H, offset, pad):
     assert (got - ref).abs().max().item() <= 2.0 ** -21 * max(1.0, ref.abs().max().item())
 
 
+@pytest.mark.parametrize("B,n_opt,t,t0,H", [(1, 1, 4100, 0, 64), (1, 2, 4100, 4095, 64), (2, 3, 257, 1, 96),
+                                            (1, 200, 9, 0, 40), (1, 70, 37, 2, 32), (700, 3, 6, 0, 16)])
+def test_readout_long_rows(gpu_lib, B, n_opt, t, t0, H):
+    """Rows whose tokens are shared out over workgroups: a token more than the chunks hold, five tokens left of many,
+    more chunks than a logit has lanes, one to 64 lanes per logit, and so many rows that none is cut."""
+    from opendecider_amd import kernels
+    g = torch.Generator().manual_seed(B + n_opt + t + H)
+    h = torch.randn(B * n_opt * t, H, generator=g).to(torch.bfloat16)
+    w = (1.0 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16)
+    head, none = torch.randn(H, generator=g) / H ** 0.5, torch.tensor(-0.2)
+    print(f"readout rows B={B} n_opt={n_opt} t={t} t0={t0} H={H}", flush=True)
+    got = kernels.readout(h.to(DEV), w.to(DEV), head.to(DEV), none.to(DEV), 1e-6, 1.3, B, n_opt, t, t0).cpu()
+    hn = od.rmsnorm(h, w, 1e-6).double().reshape(B, n_opt, t, H)[:, :, t0:].mean(2)
+    ref = torch.log_softmax(torch.cat([hn @ head.double(), none.double().expand(B, 1)], 1) / 1.3, -1)
+    assert (got - ref).abs().max().item() <= 2.0 ** -21 * max(1.0, ref.abs().max().item())
+
+
 T1_MULTIPLE = 2.0
 
 
