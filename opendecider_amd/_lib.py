@@ -156,6 +156,17 @@ def require_gpu(*tensors, name: str) -> None:
                                "opendecider_amd has no CPU path")
 
 
+def unwatched(*tensors: torch.Tensor) -> bool:
+    """True where a kernel may stand in for torch operators on these tensors: nothing records or transforms them (a
+    gradient, a forward-mode tangent, torch.func, a dispatch mode, tracing or compilation, a tensor subclass), which
+    a raw pointer would pass by."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0 or \
+            torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack():
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad) for t in tensors)
+
+
 def bf16_bits(t: torch.Tensor) -> torch.Tensor:
     if t.dtype != torch.bfloat16:
         raise TypeError(f"expected bfloat16, got {t.dtype}")

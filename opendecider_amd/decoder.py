@@ -20,7 +20,7 @@ from dataclasses import dataclass, field
 
 import torch
 
-from . import kernels
+from . import _lib, kernels
 from .kv_cache import GDNState, HybridState, Int8KVCache, StateKV
 
 
@@ -480,7 +480,7 @@ class DenseDecoder:
     def _embed(self, ids: torch.Tensor) -> torch.Tensor:
         """The tokens' embeddings, gathered straight into the residual buffer of their workspace (returned)."""
         h = self.workspace(ids.numel())["h"][0]
-        if self.embed.dtype == h.dtype and not self.embed.requires_grad:
+        if self.embed.dtype == h.dtype and not self.embed.requires_grad and _lib.unwatched(self.embed):
             return torch.index_select(self.embed, 0, ids.reshape(-1), out=h)
         return h.copy_(self.embed.index_select(0, ids.reshape(-1)))
 
@@ -621,9 +621,7 @@ class DenseDecoder:
         divided by the decision temperature (softmax(logits / T), decider.py:255-257), log-softmax per request:
         (B, n_opt + 1) fp32. The RMSNorm factor is the correctly rounded one (a float64 mean of squares, as
         od_rmsnorm_quant computes it); with cfg.norm_offset the zero-centred norm bf16((h * r) * (1 + w))."""
-        params = (h, self.final_norm, self.head, self.none_logit)
-        if h.dtype == self.final_norm.dtype == torch.bfloat16 and h.is_cuda and h.dim() == 2 and h.stride(1) == 1 \
-                and self.temperature != 0 and not (torch.is_grad_enabled() and any(x.requires_grad for x in params)):
+        if self._readout_in_kernel(h, B * n_opt * t):
             t0, t1, _ = slice(0 if pool_last is None else t - pool_last, None).indices(t)
             if t0 < t1:
                 return kernels.readout(h, self.final_norm, self.head, self.none_logit, self._eps32, self.temperature, B,
@@ -641,6 +639,18 @@ class DenseDecoder:
         return torch.log_softmax(logits / self.temperature, -1)
 
     def positions(self, T: int, R: int, t: int) -> torch.Tensor:
+    def _readout_in_kernel(self, h: torch.Tensor, rows: int) -> bool:
+        """Whether od_readout takes a readout: the operands it is written for (bf16 rows that do not overlap, fp32 head
+        and scalar none logit, a temperature with an fp32 reciprocal) and nothing that watches them. Everything else
+        goes through torch operators."""
+        H = h.shape[-1]
+        return _lib.unwatched(h, self.final_norm, self.head, self.none_logit) and \
+            h.is_cuda and h.dim() == 2 and h.shape[0] == rows > 0 and h.stride(1) == 1 and \
+            (rows == 1 or h.stride(0) >= H) and h.dtype == self.final_norm.dtype == torch.bfloat16 and \
+            self.head.dtype == self.none_logit.dtype == torch.float32 and self.none_logit.numel() == 1 and \
+            self.final_norm.shape == self.head.shape == (H,) and \
+            2.0 ** -100 <= abs(self.temperature) <= 2.0 ** 100
+
         if T + t > self.cos.shape[0]:
             raise ValueError(f"positions up to {T + t} exceed the rotary tables ({self.cos.shape[0]})")
         return (T + torch.arange(t, dtype=torch.int32)).repeat(R).to(self.dev)

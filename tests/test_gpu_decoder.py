@@ -344,6 +344,46 @@ def test_readout_long_rows(gpu_lib, B, n_opt, t, t0, H):
     assert (got - ref).abs().max().item() <= 2.0 ** -21 * max(1.0, ref.abs().max().item())
 
 
+def test_readout_watched_operands(gpu_lib):
+    """What a raw pointer would pass by or misread goes through torch operators, as any readout did once: forward-mode
+    tangents, torch.func, traces, reverse mode, rows that share memory (stride 0), a bf16 none logit."""
+    import torch.autograd.forward_ad as fwd
+    cfg, w, emb, states, ids, dec, gs = _setup(CASES[0][1], *CASES[0][2:])
+    B, n_opt, t, H = 2, 3, 4, dec.head.numel()
+    g = torch.Generator().manual_seed(5)
+    h = torch.randn(B * n_opt * t, H, generator=g).to(torch.bfloat16).to(DEV)
+    d = torch.randn(H, generator=g).to(DEV)
+    head, none = dec.head, dec.none_logit
+
+    def out(hd):
+        dec.head = hd
+        try:
+            return dec.readout(h, B, n_opt, t)
+        finally:
+            dec.head = head
+
+    want = out(head)
+    x = head.clone().requires_grad_()
+    o = out(x)
+    rows = [torch.autograd.grad(y, x, retain_graph=True)[0] for y in o.reshape(-1)]
+    tangent = (torch.stack(rows) @ d).view_as(o)  # the Jacobian by reverse mode, times d
+    with fwd.dual_level():
+        got = fwd.unpack_dual(out(fwd.make_dual(head, d))).tangent
+    assert got is not None and (got - tangent).abs().max().item() <= 1e-5 * tangent.abs().max().item()
+    assert (torch.func.jvp(out, (head,), (d,))[1] - tangent).abs().max().item() <= 1e-5 * tangent.abs().max().item()
+    heads = torch.stack([head, head + d])
+    each = torch.stack([out(a) for a in heads])
+    assert (torch.func.vmap(out)(heads) - each).abs().max().item() <= 1e-5
+    traced = torch.jit.trace(out, (head,), check_trace=False)
+    assert (traced(head + d) - each[1]).abs().max().item() <= 1e-5
+    same = dec.readout(h[:1].expand(B * n_opt * t, H), B, n_opt, t)
+    assert (same - dec.readout(h[:1].repeat(B * n_opt * t, 1), B, n_opt, t)).abs().max().item() <= 1e-5
+    dec.none_logit = none.to(torch.bfloat16)
+    low = dec.readout(h, B, n_opt, t)
+    dec.none_logit = none
+    assert low.dtype == torch.float32 and (low - want).abs().max().item() <= 2.0 ** -7 * (1.0 + none.abs().item())
+
+
 T1_MULTIPLE = 2.0
 
 
