@@ -593,7 +593,8 @@ class DenseDecoder:
         if key not in self._rows:
             pos = torch.cat([T + n + torch.arange(t, dtype=torch.int32) for n in qc.qlen for _ in range(n_opt)])
             row_q = torch.arange(G, dtype=torch.int32).repeat_interleave(n_opt)
-            self._rows[key] = (pos.to(self.dev), *kernels.row_start_of([n_opt] * G, self.dev), row_q.to(self.dev))
+            self._rows[key] = (pos.to(self.dev), *kernels.row_start_of([n_opt] * G, self.dev, kept=True),
+                               row_q.to(self.dev))
         pos, row_start, max_rows, row_q = self._rows[key]
         ws = self.workspace(R * t)
         h, mid = ws["h"]
@@ -638,7 +639,6 @@ class DenseDecoder:
         logits = torch.cat([pooled @ self.head, self.none_logit.expand(B, 1)], 1)
         return torch.log_softmax(logits / self.temperature, -1)
 
-    def positions(self, T: int, R: int, t: int) -> torch.Tensor:
     def _readout_in_kernel(self, h: torch.Tensor, rows: int) -> bool:
         """Whether od_readout takes a readout: the operands it is written for (bf16 rows that do not overlap, fp32 head
         and scalar none logit, a temperature with an fp32 reciprocal) and nothing that watches them. Everything else
@@ -651,6 +651,7 @@ class DenseDecoder:
             self.final_norm.shape == self.head.shape == (H,) and \
             2.0 ** -100 <= abs(self.temperature) <= 2.0 ** 100
 
+    def positions(self, T: int, R: int, t: int) -> torch.Tensor:
         if T + t > self.cos.shape[0]:
             raise ValueError(f"positions up to {T + t} exceed the rotary tables ({self.cos.shape[0]})")
         return (T + torch.arange(t, dtype=torch.int32)).repeat(R).to(self.dev)
@@ -673,7 +674,7 @@ class DenseDecoder:
         key = ("prefill", n0, B, S)
         if key not in self._rows:
             pos = (n0 + torch.arange(S, dtype=torch.int32)).repeat(B).to(self.dev)
-            row_start = kernels.row_start_of([1] * B, self.dev)[0] if (n0 > 0 and B > 1) else None
+            row_start = kernels.row_start_of([1] * B, self.dev, kept=True)[0] if (n0 > 0 and B > 1) else None
             self._rows[key] = (pos, row_start)
         return self._rows[key]
 
@@ -714,7 +715,7 @@ class DenseDecoder:
         key = (T, B, n_opt, t)
         if key not in self._rows:
             pos = self.positions(T, B * n_opt, t)
-            row_start, max_rows = kernels.row_start_of([n_opt] * B, self.dev)
+            row_start, max_rows = kernels.row_start_of([n_opt] * B, self.dev, kept=True)
             self._rows[key] = (pos, row_start, max_rows)
         return self._rows[key]
 

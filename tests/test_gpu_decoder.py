@@ -384,6 +384,31 @@ def test_readout_watched_operands(gpu_lib):
     assert low.dtype == torch.float32 and (low - want).abs().max().item() <= 2.0 ** -7 * (1.0 + none.abs().item())
 
 
+def test_kept_row_offsets_serve_any_stream(gpu_lib, monkeypatch):
+    """The layout a decoder keeps per shape is in place when it is returned, so that a later call on another stream,
+    which knows nothing of the one that built it, reads it whole: also with other work (here a second thread's, put
+    between the layout's two tensors) ahead of it on its stream."""
+    cfg, w, emb, states, ids, dec, gs = _setup(CASES[0][1], *CASES[0][2:])
+    positions = dec.positions
+
+    def busy(*args):
+        pos = positions(*args)
+        torch.cuda._sleep(100_000_000)
+        return pos
+
+    monkeypatch.setattr(dec, "positions", busy)
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        old = torch.full((16,), -1, dtype=torch.int32, device=DEV)
+        side.synchronize()
+        del old  # what the offsets may be given the memory of
+        row_start = dec.row_layout(70, 9, 5, 4)[1]
+    with torch.cuda.stream(other):
+        seen = row_start.cpu()
+    side.synchronize()
+    assert torch.equal(seen, 5 * torch.arange(10, dtype=torch.int32))
+
+
 T1_MULTIPLE = 2.0
 
 
