@@ -176,3 +176,17 @@ def test_left_pads_and_stream_order(gpu_lib, B, H, G, T, S, DK, DV, pads, causal
     got = lse.cpu()
     assert torch.equal(got.isinf(), ref.isinf())
     assert (got - ref)[~ref.isinf()].abs().max().item() <= 1e-4 if (~ref.isinf()).any() else True
+
+
+@pytest.mark.parametrize("B,H,G,T,S,D,pads", [(9, 16, 1, 240, 720, 128, None), (9, 16, 1, 236, 940, 128, [130] * 9),
+                                              (5, 16, 1, 237, 500, 256, [64, 0, 300, 1, 63])])
+def test_stream_order_over_more_workgroups_than_cus(gpu_lib, B, H, G, T, S, D, pads):
+    """More than 256 workgroups of causal queries that are a fourth to a half of the keys: the tiles of all streams side
+    by side, heaviest first, with 1 and 2 halves."""
+    q, k, v, _ = make(B * 100 + S + D, B, H, G, T, S, D, D, False)
+    kv = None if pads is None else torch.arange(S)[None, :] >= torch.tensor(pads)[:, None]
+    out, lse = run(q, k, v, kv, True)
+    ob, lb, bound = oa.wide_attention_blocked(q, k, v, D ** -0.5, kv, True, with_bound=True)
+    check_vs_blocked(out.cpu().float(), ob, bound, f"stream order T={T} S={S}")
+    ref = oa.attention(q, k, v, D ** -0.5, kv, True, dtype=torch.float64)[1].float()
+    assert (lse.cpu() - ref).abs().max().item() <= 1e-4
