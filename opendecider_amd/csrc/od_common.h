@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/od_mi355x.h"
 
 #define OD_WAVE 64
@@ -273,4 +275,18 @@ __device__ __forceinline__ int8_t od_q8_one(float v, float scale, float inv) {
   float t = od_q8_fast(v, inv, d);
   if (d >= kOdTieEdge) t = od_q8_exact(v, scale);
   return (int8_t)(__float_as_uint(t) & 0xffu);
+}
+
+// Compute units of the current device, rounded down to a multiple of 8 (whole XCDs), cached per device
+inline int od_cu_count() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
+    n -= n % 8;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }

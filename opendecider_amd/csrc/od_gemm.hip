@@ -34,7 +34,6 @@
 // sustain about 3.0-3.1 of the 5.0 POP/s peak (the clock drops to about 1.9-2.1 GHz under that load; with constant
 // operands the same loop reaches 4.9 POP/s at 2.38 GHz).
 // int32 accumulation is exact for K < 133,144 (|acc| <= 127^2 K < 2^31), so any correct GEMM is bit-exact.
-#include <atomic>
 #include <type_traits>
 
 #include "od_common.h"
@@ -829,20 +828,6 @@ __global__ __launch_bounds__(kSmWaves * 64, 1) void w8a8_gemm_small_kernel(GemmA
 
 namespace {
 
-// compute units of the current device, rounded down to a multiple of 8 (whole XCDs), cached per device
-int cu_count() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
-    n -= n % 8;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 struct Tiling {
   int bm, bn;
   int64_t tiles_m, tiles_n;
@@ -863,7 +848,7 @@ constexpr double kRel128x128 = 0.53, kRel128x128Pair = 0.60;
 Tiling tiling_of(int64_t M, int64_t N, bool small) {
   const struct { int bm, bn; double cost; } cand[4] = {
       {256, 256, 1.0}, {256, 192, 0.84}, {128, 256, 0.68}, {128, 128, kRel128x128}};
-  const int64_t cus = cu_count();
+  const int64_t cus = od_cu_count();
   Tiling best{256, 256, 0, 0, 1.0};
   double best_cost = 0.0;
   for (const auto& c : cand) {
@@ -899,10 +884,10 @@ struct SplitPlan {
 // 31 us, in two of 32 42; 256 x 6144 x 4096 in one round of 96 18.5, in two of 64 26.
 constexpr int64_t kSmallMaxM = 512;
 bool small_m(int64_t M, int64_t N) {
-  return M <= kSmallMaxM && ((M + kSmBM - 1) / kSmBM) * ((N + 63) / 64) <= 2 * (int64_t)cu_count();
+  return M <= kSmallMaxM && ((M + kSmBM - 1) / kSmBM) * ((N + 63) / 64) <= 2 * (int64_t)od_cu_count();
 }
 int small_bn(int64_t M, int64_t N) {
-  const int64_t tm = (M + kSmBM - 1) / kSmBM, cus = cu_count();
+  const int64_t tm = (M + kSmBM - 1) / kSmBM, cus = od_cu_count();
   int best = 64;
   double t = 1e30;
   for (const int bn : {64, 32, 96}) {
@@ -921,7 +906,7 @@ SplitPlan split_plan(int64_t M, int64_t N, int64_t K) {
   const SplitPlan none{1, nk, 0, 0};
   if (small_m(M, N)) return none;  // the small-M kernel splits K inside its workgroups
   const Tiling t = tiling_of(M, N, false);
-  const int64_t ntiles = t.tiles_m * t.tiles_n, cus = cu_count();
+  const int64_t ntiles = t.tiles_m * t.tiles_n, cus = od_cu_count();
   if (ntiles * 2 > cus || nk < 4) return none;
   const double t_stage = 1.2 * t.rel;  // us per k-tile stage of one tile
   const double base = nk * t_stage;
@@ -1034,7 +1019,7 @@ int gemm_launch(const GemmArgs& p0, bool swiglu, hipStream_t st, const SplitPlan
   // persistent workgroups: one per CU (the kernel's LDS admits one; two of the 128 x 128 tile's), each looping over
   // tiles bid + i * grid
   const int64_t ntiles = tiles_m * tiles_n;
-  const int64_t gmax = (t.bm == 128 && t.bn == 128 ? 2 : 1) * cu_count();
+  const int64_t gmax = (t.bm == 128 && t.bn == 128 ? 2 : 1) * od_cu_count();
   dim3 grid((unsigned)(ntiles <= gmax ? ntiles : gmax)), block(kThreads);
   enum { kFast, kGeneral, kWide };
   auto launch = [&](auto BMc, auto BNc, auto ACCc, auto GENc, auto SWc, auto WIc) {
@@ -1063,7 +1048,7 @@ int gemm_launch(const GemmArgs& p0, bool swiglu, hipStream_t st, const SplitPlan
       // else two workgroups per CU on 2 stages each
       if constexpr (!decltype(ACCc)::value) {
         if (variant == kWide) {
-          if (ntiles <= cu_count() && p.kt_per >= 24)
+          if (ntiles <= od_cu_count() && p.kt_per >= 24)
             w8a8_gemm_kernel<128, 128, false, false, decltype(SWc)::value, true, 4><<<grid, block, 0, st>>>(p);
           else
             launch(H{}, H{}, ACCc, std::false_type{}, SWc, std::true_type{});

@@ -723,14 +723,18 @@ extern "C" int od_wide_attn(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t
   WideArgs a{q, k, v, kvalid, out, lse, sqb, sqh, sqt, skb, skg, sks, svb, svg, svs, sob, soh, sot, smb,
              (int)H, (int)G, (int)T, (int)S, (int)DK, (int)rep, causal ? 1 : 0, scale * 1.4426950408889634f, 0, 0};
   // The tiles of all streams side by side (wide_tile) where a tile's work varies, causal over at most four times the
-  // queries' keys: with an XCD's contiguous range cutting a (batch, group) (B G not a multiple of 8) at every size (3
-  // left-padded states of 1537 tokens, 16 / 4 heads of 256, with the skipped blocks 146 -> 95 us; 1 x 32768 of the same
-  // heads 8.8 -> 5.9 ms), else with up to 96 MB of K and V (8 x 2048 tokens, 32 / 8 heads of 128: 191 -> 174 us;
-  // 2 x 1000: 43 -> 37). Above it an XCD reads all its streams' K/V at once and misses the caches (8 x 4000 tokens
-  // after 3900, 32 / 8 heads: 1613 us in ranges, 1736 side by side), as over more keys, where the tiles are alike
-  // (3 x 1000 tokens after 8000, 12 / 4 heads: 141 and 146 us).
-  a.by_tile = causal && 4 * T >= S && (B * G % 8 != 0 || B * G * S * (DK + DV) <= (48 << 20)) &&
-              tiles * B * G <= 0x3fffffff;
+  // queries' keys, and the CUs take more than one round (a single round ends with its heaviest tile in any order, and
+  // the ranges read fewer streams per L2: 1 x 500 tokens after 1450, 28 / 7 heads of 128, 112 workgroups, 44.6 us in
+  // ranges, 49.5 side by side; 266 workgroups of the same heads 42.8 and 41.2): with an XCD's contiguous range cutting
+  // a (batch, group) (B G not a multiple of 8) at every size (3 left-padded states of 1537 tokens, 16 / 4 heads of 256,
+  // with the skipped blocks 146 -> 95 us; 1 x 32768 of the same heads 8.8 -> 5.9 ms), else with up to 96 MB of K and V
+  // (8 x 2048 tokens, 32 / 8 heads of 128: 191 -> 174 us; 2 x 1000: 43 -> 37). Above it an XCD reads all its streams'
+  // K/V at once and misses the caches (8 x 4000 tokens after 3900, 32 / 8 heads: 1613 us in ranges, 1736 side by side),
+  // as over more keys, where the tiles are alike (3 x 1000 tokens after 8000, 12 / 4 heads: 141 and 146 us). Where it
+  // still loses: 270 to 320 workgroups of 3 streams, queries over their own keys, 3 to 4%.
+  const int64_t groups = tiles * B * G * (DV == 256 && DK > 128 ? 2 : 1);  // workgroups, 2 per tile in halves
+  a.by_tile = causal && 4 * T >= S && groups > od_cu_count() && groups <= 0x7fffffff &&
+              (B * G % 8 != 0 || B * G * S * (DK + DV) <= (48 << 20));
   dim3 grid((unsigned)tiles, (unsigned)(B * G));
   hipStream_t st = (hipStream_t)stream;
   const int dkp = DK <= 64 ? 64 : DK <= 128 ? 128 : DK <= 256 ? 256 : 512;
