@@ -112,6 +112,7 @@ __device__ __forceinline__ float silu_bf16(float g) {
 //           its rounding; rsq within 1 ulp, so its bf16 is right unless the low half lies within 4 ulps of the midpoint;
 //           else (1 wave in 200) float64
 constexpr int kTok = 16;
+constexpr int kPrepChan = 8;
 constexpr int kPrepThreads = 256;
 
 __device__ __forceinline__ float group_sum(float v, int G) {
@@ -125,45 +126,132 @@ __device__ __forceinline__ float group_sum(float v, int G) {
   return v;
 }
 
+// l2norm of a q / k head's channels (yw, bf16 pairs; G lanes a head): squares rounded to bf16, their exact sum rounded
+// to bf16, + eps, rsqrt and the product each rounded to bf16 (torch's bf16 arithmetic, with a correctly rounded rsqrt).
+// Every lane of the wave takes part, a lane of no q / k channel (mine false) with any values.
 template <int NCH>
-__global__ __launch_bounds__(kPrepThreads, NCH == 8 ? 3 : 1) void gdn_prep_kernel(PrepArgs p) {
-  constexpr int NW = NCH / 2;  // words of bf16 pairs
-  __shared__ uint16_t stab[2 * kSiluHalf];
-  for (int i = threadIdx.x; i < (int)(2 * kSiluHalf); i += blockDim.x) stab[i] = od_silu_table_entry(i);
-  __syncthreads();
-  const int64_t ntile = (p.L + kTok - 1) / kTok;
-  const int64_t s = blockIdx.x / ntile, t0 = (blockIdx.x % ntile) * kTok;
-  const int64_t m_s = s * p.L;  // first token of the sequence
-  const int tid = threadIdx.x;
-  const int c0 = ((int)blockIdx.y * (int)blockDim.x + tid) * NCH;
-  const bool on = c0 < p.C;
-  const int64_t st = p.seq_state ? (int64_t)p.seq_state[s] : s;
-  const bool st_ok = p.conv_in != nullptr && st >= 0 && st < p.n_states;
-  const int kd = p.n_k * p.dk;
-  const int G = p.dk / NCH;  // lanes per head (a power of two <= 64)
-  const int tn = (int)min((int64_t)kTok, p.L - t0);
-  // real tokens of the sequence (clamped into [0, L]); tokens at or past it are right pads
-  const int64_t len = p.seq_len ? min(max((int64_t)p.seq_len[s], (int64_t)0), p.L) : p.L;
+__device__ __forceinline__ void prep_l2norm(uint32_t (&yw)[NCH / 2], bool mine, int G) {
+  float y[NCH], sq[NCH];
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NCH / 2; ++i) {
+    y[2 * i] = __uint_as_float(yw[i] << 16);
+    y[2 * i + 1] = __uint_as_float(yw[i] & 0xffff0000u);
+  }
+#pragma unroll
+  for (int i = 0; i < NCH; i += 2) {
+    sq[i] = y[i] * y[i];
+    sq[i + 1] = y[i + 1] * y[i + 1];
+    od_bfr2(sq[i], sq[i + 1]);
+    ss += sq[i] + sq[i + 1];
+  }
+  ss = group_sum(ss, G);
+  float sb = ss * (1.0f - 0x1p-20f), sh = ss * (1.0f + 0x1p-20f);
+  od_bfr2(sb, sh);
+  float den = bf(sb + 1e-6f);
+  float inv = __builtin_amdgcn_rsqf(den);
+  const bool slow = !(sb == sh) || ((__float_as_uint(inv) & 0xffffu) - 0x7ffcu) <= 8u;
+  if (__builtin_expect(__any(slow && mine), 0)) {
+    double sd = 0.0;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) sd += (double)sq[i];
+    for (int o = G / 2; o > 0; o >>= 1) sd += __shfl_xor(sd, o, OD_WAVE);
+    den = bf(bf((float)sd) + 1e-6f);
+    inv = (float)(1.0 / sqrt((double)den));
+  }
+  inv = bf(inv);
+  if (mine) {
+#pragma unroll
+    for (int i = 0; i < NCH / 2; ++i) yw[i] = od_pack_bf16x2(y[2 * i] * inv, y[2 * i + 1] * inv);
+  }
+}
 
+// The gates of a tile's tokens (first channel block): thread i takes (token i / n_v, value head i % n_v). A right pad
+// gets beta = 0 and g = -0, what b = a = -inf give (sigmoid(-inf) = 0, softplus(-inf) = 0): the state passes through it
+// unchanged (e^g = 1, no write)
+__device__ __forceinline__ void prep_gates(const PrepArgs& p, int64_t m0, int64_t t0, int tn, int64_t len) {
+  for (int i = blockIdx.y == 0 ? (int)threadIdx.x : tn * p.n_v; i < tn * p.n_v; i += blockDim.x) {
+    const int64_t m = m0 + i / p.n_v;
+    const int hh = i % p.n_v;
+    if (t0 + i / p.n_v >= len) {
+      p.beta[m * p.n_v + hh] = 0.0f;
+      p.g[m * p.n_v + hh] = -0.0f;
+      continue;
+    }
+    const uint16_t* row = p.proj + m * p.ldp + p.C + (int64_t)p.n_v * p.dv;
+    const float b = od_bf16_to_f32(row[hh]), a = od_bf16_to_f32(row[p.n_v + hh]);
+    p.beta[m * p.n_v + hh] = od_sigmoid_bf16(b);
+    const float e = (float)exp((double)od_bf16_to_f32(p.A_log[hh]));
+    const float x = (float)((double)a + (double)od_bf16_to_f32(p.dt_bias[hh]));
+    const float sp = x > 20.0f ? x : (float)log1p(exp((double)x));
+    p.g[m * p.n_v + hh] = (float)(-((double)e * (double)sp));
+  }
+}
+
+// A thread's place in the pass: its tile of `tok` tokens of a sequence and its NCH channels from c0 on
+template <int NCH>
+struct PrepPlace {
+  int64_t s, t0, m_s;  // sequence, first token of the tile in it, first token of the sequence
+  int64_t st, len;     // state; real tokens of the sequence (clamped into [0, L]): tokens at or past it are right pads
+  int c0, tn;          // first channel, tokens of the tile
+  bool on, qk, st_ok;  // a channel, a q / k channel, a state to read
+
+  __device__ __forceinline__ PrepPlace(const PrepArgs& p, int tok) {
+    const int64_t ntile = (p.L + tok - 1) / tok;
+    s = blockIdx.x / ntile;
+    t0 = (blockIdx.x % ntile) * tok;
+    m_s = s * p.L;
+    st = p.seq_state ? (int64_t)p.seq_state[s] : s;
+    st_ok = p.conv_in != nullptr && st >= 0 && st < p.n_states;
+    len = p.seq_len ? min(max((int64_t)p.seq_len[s], (int64_t)0), p.L) : p.L;
+    c0 = ((int)blockIdx.y * (int)blockDim.x + (int)threadIdx.x) * NCH;
+    tn = (int)min((int64_t)tok, p.L - t0);
+    on = c0 < p.C;
+    qk = on && c0 < 2 * p.n_k * p.dk;
+  }
   // row r of full = [state (3 rows) ; the sequence's tokens]: full[r] = state row r (r < 3) or token r - 3, as words of
   // bf16 pairs
-  auto load_full = [&](int64_t r, uint32_t (&x)[NW]) {
+  __device__ __forceinline__ void row(const PrepArgs& p, int64_t r, uint32_t (&x)[NCH / 2]) const {
     const uint16_t* src = nullptr;
     if (r >= kConvTaps - 1) src = p.proj + (m_s + r - (kConvTaps - 1)) * p.ldp + c0;
     else if (st_ok) src = p.conv_in + (st * (kConvTaps - 1) + r) * p.C + c0;
 #pragma unroll
-    for (int i = 0; i < NW; i += 4) {
+    for (int i = 0; i < NCH / 2; i += 4) {
       const uint4 v = src ? *reinterpret_cast<const uint4*>(src + 2 * i) : make_uint4(0, 0, 0, 0);
       x[i] = v.x; x[i + 1] = v.y; x[i + 2] = v.z; x[i + 3] = v.w;
     }
-  };
-  auto unpack = [](const uint32_t (&x)[NW], float (&f)[NCH]) {
+  }
+  // whether this tile writes the new conv state, the 3 rows of full that end at the last real token (rows len .. len +
+  // 2): the tile of that token (the first tile of a sequence with no real token)
+  __device__ __forceinline__ bool writes_state(const PrepArgs& p, int tok) const {
+    return p.conv_out && on && (len == 0 ? t0 == 0 : (len - 1) / tok == t0 / tok);
+  }
+  __device__ __forceinline__ uint16_t* state_row(const PrepArgs& p, int j) const {
+    return p.conv_out + (s * (kConvTaps - 1) + j) * p.C + c0;
+  }
+  // this thread's outputs of token t
+  __device__ __forceinline__ uint16_t* out(const PrepArgs& p, int64_t t) const {
+    const int kd2 = 2 * p.n_k * p.dk;
+    const int64_t m = m_s + t;
+    return qk ? p.qk + m * (int64_t)kd2 + c0 : p.v + m * (int64_t)(p.n_v * p.dv) + (c0 - kd2);
+  }
+  static __device__ __forceinline__ void put(uint16_t* dst, const uint32_t (&x)[NCH / 2]) {
 #pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      f[2 * i] = __uint_as_float(x[i] << 16);
-      f[2 * i + 1] = __uint_as_float(x[i] & 0xffff0000u);
-    }
-  };
+    for (int i = 0; i < NCH / 2; i += 4)
+      *reinterpret_cast<uint4*>(dst + 2 * i) = make_uint4(x[i], x[i + 1], x[i + 2], x[i + 3]);
+  }
+};
+
+__global__ __launch_bounds__(kPrepThreads, 3) void gdn_prep_kernel(PrepArgs p) {
+  constexpr int NCH = kPrepChan, NW = NCH / 2;  // words of bf16 pairs
+  __shared__ uint16_t stab[2 * kSiluHalf];
+  for (int i = threadIdx.x; i < (int)(2 * kSiluHalf); i += blockDim.x) stab[i] = od_silu_table_entry(i);
+  __syncthreads();
+  const PrepPlace<NCH> at(p, kTok);
+  const int64_t t0 = at.t0;
+  const int c0 = at.c0, tn = at.tn;
+  const int G = p.dk / NCH;  // lanes per head (a power of two <= 64)
+  auto load_full = [&](int64_t r, uint32_t (&x)[NW]) { at.row(p, r, x); };
   auto widen = [](const uint32_t (&x)[NW], double (&f)[NCH]) {
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
@@ -176,7 +264,7 @@ __global__ __launch_bounds__(kPrepThreads, NCH == 8 ? 3 : 1) void gdn_prep_kerne
   uint32_t xr[2][NW];  // the rows of this token and the next, raw: loads go out two tokens ahead
 #pragma unroll
   for (int i = 0; i < NW; ++i) xr[0][i] = xr[1][i] = 0u;
-  if (on) {
+  if (at.on) {
 #pragma unroll
     for (int i = 0; i < NCH; i += 2) {  // two channels of four taps: 16 bytes
       const uint4 v = *reinterpret_cast<const uint4*>(p.conv_w + (int64_t)(c0 + i) * kConvTaps);
@@ -205,26 +293,20 @@ __global__ __launch_bounds__(kPrepThreads, NCH == 8 ? 3 : 1) void gdn_prep_kerne
       wa[i] = wb[i] = wc[i] = 0.0;
     }
   }
-  // the new conv state is the 3 rows of [state ; tokens] that end at the last real token (rows len .. len + 2), written
-  // by the tile of that token (the first tile of a sequence with no real token)
-  if (p.conv_out && on && (len == 0 ? t0 == 0 : (len - 1) / kTok == t0 / kTok)) {
+  if (at.writes_state(p, kTok)) {
 #pragma unroll
     for (int j = 0; j < kConvTaps - 1; ++j) {
       uint32_t x[NW];
-      load_full(len + j, x);
-#pragma unroll
-      for (int i = 0; i < NW; i += 4)
-        *reinterpret_cast<uint4*>(p.conv_out + (s * (kConvTaps - 1) + j) * p.C + c0 + 2 * i) =
-            make_uint4(x[i], x[i + 1], x[i + 2], x[i + 3]);
+      load_full(at.len + j, x);
+      at.put(at.state_row(p, j), x);
     }
   }
 
-  const bool qk_chan = on && c0 < 2 * kd;
   auto token = [&](int tt, const double (&x0)[NCH], const double (&x1)[NCH], const double (&x2)[NCH],
                    double (&x3)[NCH], uint32_t (&raw)[NW]) {
-    const int64_t t = t0 + tt, m = m_s + t;
+    const int64_t t = t0 + tt;
     widen(raw, x3);
-    if (on && tt + 2 < tn) load_full(t + kConvTaps + 1, raw);
+    if (at.on && tt + 2 < tn) load_full(t + kConvTaps + 1, raw);
     uint32_t yw[NW], gw[NW];
     od_u16x2 far = {0, 0};  // the largest distance of 2 |g|'s pattern above the smallest that the table steps cover
 #pragma unroll
@@ -252,52 +334,14 @@ __global__ __launch_bounds__(kPrepThreads, NCH == 8 ? 3 : 1) void gdn_prep_kerne
       far = __builtin_elementwise_max(far, (od_u16x2)(d - (uint16_t)0x200));
     }
     constexpr uint16_t kFar = 2 * kSiluHi - 0x200;  // |g| >= 16, infinite or NaN; |g| < 2^-125 wraps past it
-    if (__builtin_expect((far.x >= kFar || far.y >= kFar) && on, 0)) {
+    if (__builtin_expect((far.x >= kFar || far.y >= kFar) && at.on, 0)) {
       asm volatile("");  // a branch, not selects
 #pragma unroll
       for (int i = 0; i < NW; ++i)
         yw[i] = od_pack_bf16x2(silu_bf16(__uint_as_float(gw[i] << 16)), silu_bf16(__uint_as_float(gw[i] & 0xffff0000u)));
     }
-    // l2norm of the q and k heads: squares rounded to bf16, their exact sum rounded to bf16, + eps, rsqrt and the
-    // product each rounded to bf16 (torch's bf16 arithmetic, with a correctly rounded rsqrt)
-    if (__builtin_amdgcn_ballot_w64(qk_chan)) {
-      float y[NCH];
-      unpack(yw, y);
-      float ss = 0.0f;
-      float sq[NCH];
-#pragma unroll
-      for (int i = 0; i < NCH; i += 2) {
-        sq[i] = y[i] * y[i];
-        sq[i + 1] = y[i + 1] * y[i + 1];
-        od_bfr2(sq[i], sq[i + 1]);
-        ss += sq[i] + sq[i + 1];
-      }
-      ss = group_sum(ss, G);
-      float sb = ss * (1.0f - 0x1p-20f), sh = ss * (1.0f + 0x1p-20f);
-      od_bfr2(sb, sh);
-      float den = bf(sb + 1e-6f);
-      float inv = __builtin_amdgcn_rsqf(den);
-      const bool slow = !(sb == sh) || ((__float_as_uint(inv) & 0xffffu) - 0x7ffcu) <= 8u;
-      if (__builtin_expect(__any(slow && qk_chan), 0)) {
-        double sd = 0.0;
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) sd += (double)sq[i];
-        for (int o = G / 2; o > 0; o >>= 1) sd += __shfl_xor(sd, o, OD_WAVE);
-        den = bf(bf((float)sd) + 1e-6f);
-        inv = (float)(1.0 / sqrt((double)den));
-      }
-      inv = bf(inv);
-      if (qk_chan) {
-#pragma unroll
-        for (int i = 0; i < NW; ++i) yw[i] = od_pack_bf16x2(y[2 * i] * inv, y[2 * i + 1] * inv);
-      }
-    }
-    if (on) {
-      uint16_t* dst = qk_chan ? p.qk + m * (int64_t)(2 * kd) + c0 : p.v + m * (int64_t)(p.n_v * p.dv) + (c0 - 2 * kd);
-#pragma unroll
-      for (int i = 0; i < NW; i += 4)
-        *reinterpret_cast<uint4*>(dst + 2 * i) = make_uint4(yw[i], yw[i + 1], yw[i + 2], yw[i + 3]);
-    }
+    if (__builtin_amdgcn_ballot_w64(at.qk)) prep_l2norm<NCH>(yw, at.qk, G);
+    if (at.on) at.put(at.out(p, t), yw);
   };
   for (int tt = 0; tt < tn; tt += 4) {
     token(tt, wa, wb, wc, wd, xr[0]);
@@ -308,27 +352,67 @@ __global__ __launch_bounds__(kPrepThreads, NCH == 8 ? 3 : 1) void gdn_prep_kerne
     if (tt + 3 >= tn) break;
     token(tt + 3, wd, wa, wb, wc, xr[1]);
   }
+  prep_gates(p, at.m_s + t0, t0, tn, at.len);
+}
 
-  // gates of the tile's tokens (first channel block): thread i takes (token i / n_v, value head i % n_v). A right pad
-  // gets beta = 0 and g = -0, what b = a = -inf give (sigmoid(-inf) = 0, softplus(-inf) = 0): the state passes
-  // through it unchanged (e^g = 1, no write)
-  for (int i = blockIdx.y == 0 ? tid : tn * p.n_v; i < tn * p.n_v; i += blockDim.x) {
-    const int64_t m = m_s + t0 + i / p.n_v;
-    const int hh = i % p.n_v;
-    if (t0 + i / p.n_v >= len) {
-      p.beta[m * p.n_v + hh] = 0.0f;
-      p.g[m * p.n_v + hh] = -0.0f;
-      continue;
-    }
-    const uint16_t* row = p.proj + m * p.ldp + p.C + (int64_t)p.n_v * p.dv;
-    const float b = od_bf16_to_f32(row[hh]), a = od_bf16_to_f32(row[p.n_v + hh]);
-    p.beta[m * p.n_v + hh] = od_sigmoid_bf16(b);
-    const float e = (float)exp((double)od_bf16_to_f32(p.A_log[hh]));
-    const float x = (float)((double)a + (double)od_bf16_to_f32(p.dt_bias[hh]));
-    const float sp = x > 20.0f ? x : (float)log1p(exp((double)x));
-    p.g[m * p.n_v + hh] = (float)(-((double)e * (double)sp));
+// The same bytes for sequences of up to kTokShort tokens, and for heads of more than 64 lanes of 8 channels (dk = 1024,
+// NCH = 16): tiles of kTokShort tokens, every row held raw, each operand converted where it is used, and the silu
+// function in place of the table. Bound by memory latency and, with many sequences, bandwidth (4096 x 1 token, 16 / 32
+// heads, with the new conv states: 528 MB in 110 us): filling a table (12 entries a thread) and widening the taps and
+// the window pay only over more tokens, and 105 VGPRs leave four waves per SIMD in place of three. 1024 sequences of 1,
+// 2, 3 and 4 tokens: 26, 35, 44 and 54 us (with the table 38, 47, 55 and 63); 256 x 24 tokens at dk = 1024 183 -> 132.
+constexpr int kTokShort = 4;
+template <int NCH>
+__global__ __launch_bounds__(kPrepThreads) void gdn_prep_short_kernel(PrepArgs p) {
+  constexpr int NW = NCH / 2;
+  const PrepPlace<NCH> at(p, kTokShort);
+  uint32_t wr[2 * NCH];            // taps: channel c has words 2 c and 2 c + 1
+  uint32_t x[kConvTaps - 1 + kTokShort][NW];  // full rows t0 .. t0 + tn + 2
+#pragma unroll
+  for (int i = 0; i < 2 * NCH; i += 4) {
+    const uint4 v = at.on ? *reinterpret_cast<const uint4*>(p.conv_w + (int64_t)at.c0 * kConvTaps + 2 * i)
+                          : make_uint4(0, 0, 0, 0);
+    wr[i] = v.x; wr[i + 1] = v.y; wr[i + 2] = v.z; wr[i + 3] = v.w;
   }
-
+#pragma unroll
+  for (int r = 0; r < kConvTaps - 1 + kTokShort; ++r) {
+    if (at.on && r < kConvTaps - 1 + at.tn) {
+      at.row(p, at.t0 + r, x[r]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) x[r][i] = 0u;
+    }
+  }
+  if (at.writes_state(p, kTokShort)) {
+#pragma unroll
+    for (int r = 0; r <= kTokShort; ++r)
+      if (at.len - at.t0 == r) {
+#pragma unroll
+        for (int j = 0; j < kConvTaps - 1; ++j) at.put(at.state_row(p, j), x[r + j]);
+      }
+  }
+#pragma unroll
+  for (int tt = 0; tt < kTokShort; ++tt) {
+    if (tt >= at.tn) break;
+    uint32_t yw[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      float acc[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        auto half = [&](uint32_t w, int hi) { return (double)__uint_as_float(hi ? w & 0xffff0000u : w << 16); };
+        uint32_t w01 = wr[4 * i + 2 * k], w23 = wr[4 * i + 2 * k + 1];
+        asm volatile("" : "+v"(w01), "+v"(w23));  // keeps the widened taps out of the registers between tokens
+        acc[k] = (float)fma(half(w23, 1), half(x[tt + 3][i], k),
+                            fma(half(w23, 0), half(x[tt + 2][i], k),
+                                fma(half(w01, 1), half(x[tt + 1][i], k), half(w01, 0) * half(x[tt][i], k))));
+      }
+      yw[i] = od_pack_bf16x2(silu_bf16(bf(acc[0])), silu_bf16(bf(acc[1])));
+    }
+    if (__builtin_amdgcn_ballot_w64(at.qk)) prep_l2norm<NCH>(yw, at.qk, p.dk / NCH);
+    if (at.on) at.put(at.out(p, at.t0 + tt), yw);
+  }
+  prep_gates(p, at.m_s + at.t0, at.t0, at.tn, at.len);
 }
 
 // ------------------------------------------------------------------------------------------------ recurrence
@@ -662,15 +746,19 @@ extern "C" int od_gdn_prep_ex(const uint16_t* proj, int64_t ldp, const uint16_t*
   if (S * L > 0x7fffffffll) return OD_ERR_SHAPE;
   PrepArgs p{proj, conv_w, conv_in, seq_state, A_log, dt_bias, qk, v, g, beta, conv_out, seq_len, ldp, S, L,
              n_states, (int)n_k, (int)n_v, (int)dk, (int)dv, (int)C};
-  const int64_t tiles = S * ((L + kTok - 1) / kTok);
   // 8 channels per thread (16-byte rows) wherever a head then fits a wave's lanes
-  const int nch = dk / 8 <= 64 ? 8 : 16;
+  const int nch = dk / kPrepChan <= 64 ? kPrepChan : kChan;
+  const bool few = nch != kPrepChan || L <= kTokShort;
+  const int64_t tok = few ? kTokShort : kTok, tiles = S * ((L + tok - 1) / tok);
   const int threads = (int)min((C / nch + 63) / 64 * 64, (int64_t)kPrepThreads);
   const dim3 grid((unsigned)tiles, (unsigned)((C / nch + threads - 1) / threads));
-  if (nch == 8)
-    gdn_prep_kernel<8><<<grid, dim3(threads), 0, (hipStream_t)stream>>>(p);
+  hipStream_t hs = (hipStream_t)stream;
+  if (nch != kPrepChan)
+    gdn_prep_short_kernel<kChan><<<grid, dim3(threads), 0, hs>>>(p);
+  else if (few)
+    gdn_prep_short_kernel<kPrepChan><<<grid, dim3(threads), 0, hs>>>(p);
   else
-    gdn_prep_kernel<16><<<grid, dim3(threads), 0, (hipStream_t)stream>>>(p);
+    gdn_prep_kernel<<<grid, dim3(threads), 0, hs>>>(p);
   return od_launch_status();
 }
 

@@ -137,6 +137,18 @@ def test_gdn_prep_padded_sequences_bit_exact(gpu_lib, S, L, n_k, n_v, lens):
     assert torch.equal(co.cpu(), new)
 
 
+@pytest.mark.parametrize("L", [1, 2, 3, 4, 5])
+def test_gdn_prep_short_sequences(gpu_lib, L):
+    """Up to the 4 tokens that the short-sequence kernel takes and one more, with values of every magnitude, states with
+    and without an entry, and 0 to L real tokens; heads of 1024 over several of its tiles."""
+    test_gdn_prep_tiles_and_special_values(gpu_lib, 3, L, 2, 4, 128, 128)
+    test_gdn_prep_tiles_and_special_values(gpu_lib, 2, L, 1, 2, 16, 16)
+    test_gdn_prep_tiles_and_special_values(gpu_lib, 3, L + 6, 1, 1, 1024, 32)
+    test_gdn_prep_bit_exact(gpu_lib, 5, L, 2, 4, True)
+    test_gdn_prep_bit_exact(gpu_lib, 3, L, 16, 32, False)
+    test_gdn_prep_padded_sequences_bit_exact(gpu_lib, L + 1, L, 2, 4, list(range(L + 1)))
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 def test_gdn_padded_continuation_keeps_each_state(gpu_lib, chunked):
     """The recurrence over right-padded sequences (gates from od_gdn_prep_ex) leaves each sequence's final state equal
