@@ -14,8 +14,10 @@
 // gdn_chunk_t, per (sequence, chunk, key head): K K^T on MFMA and T in fp32, by forward substitution in two blocks,
 // for each value head of that key head, written as bf16 hi / lo in the layout the second kernel copies straight into
 // LDS, with the vectors gamma, e^gamma, e^{gamma_C - gamma} and e^{gamma_C}. Then, chunk after chunk (the only
-// sequential part), gdn_chunk_roles (a role per wave) or gdn_chunk_state (one chunk, see the dispatch), both per
-// (sequence, value head, 64 state columns) with 16 columns per wave; gdn_chunk_state takes P from
+// sequential part), one of three kernels with 16 state columns per wave (see the dispatch): gdn_chunk_roles<false>, a
+// role per wave, per (sequence, value head, 64 columns); gdn_chunk_roles<true>, the same over one-chunk sequences that
+// keep no state, per (run of sequences, value head, 128 columns); gdn_chunk_state, one or two chunks with every wave
+// doing all of it, per (sequence, value head, 64 columns). gdn_chunk_state takes P from
 // K Q~^T on MFMA, then the products above. The state lives in the MFMA accumulators
 // (V_MFMA_F32_16X16X32_BF16, lane l: column l % 16, rows 4 (l / 16) + i of each 16 x 16 tile) and feeds the next
 // products straight from there: an accumulator tile's rows become a B operand's k-values in the order
@@ -318,7 +320,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_state_kernel(CArgs p) {
     for (int i = 0; i < 4; ++i)
       S[r][i] = has_init ? p.init[((sidx * p.n_v + h) * kDk + 16 * r + 4 * h4 + i) * p.dv + col] : 0.0f;
 
-  // chunk inputs, prefetched into registers one chunk ahead. K and V: thread (tp, part) takes tokens 2 tp and
+  // chunk inputs, loaded into registers first. K and V: thread (tp, part) takes tokens 2 tp and
   // 2 tp + 1 of one 8-wide part, so that the transposed copies are written as token pairs
   const int tp = tid & 15, kp = tid >> 4, vp = (tid >> 4) & 7;
   struct Pre {
@@ -486,24 +488,18 @@ __global__ __launch_bounds__(256) void gdn_chunk_state_kernel(CArgs p) {
           *reinterpret_cast<const uint4*>(&ob[tid >> 3][8 * (tid & 7)]);
   };
 
-  // chunk inputs are loaded two chunks ahead (two register sets, alternating)
-  Pre pa = gload(0);
-  swrite(pa);
+  // one or two chunks (see the dispatch), the second one's inputs loaded while the first is computed
+  Pre pre = gload(0);
+  swrite(pre);
   __syncthreads();
-  Pre pb = pa;
-  if (p.nchunk > 1) pb = gload(1);
-  for (int64_t c = 0; c < p.nchunk; c += 2) {
-    if (c + 2 < p.nchunk) pa = gload(c + 2);
-    compute();
-    finish(c);
-    if (c + 1 >= p.nchunk) break;
-    swrite(pb);
+  if (p.nchunk > 1) pre = gload(1);
+  compute();
+  finish(0);
+  if (p.nchunk > 1) {
+    swrite(pre);
     __syncthreads();
-    if (c + 3 < p.nchunk) pb = gload(c + 3);
     compute();
-    finish(c + 1);
-    if (c + 2 < p.nchunk) swrite(pa);
-    __syncthreads();
+    finish(1);
   }
   if (p.final_state) {
 #pragma unroll
@@ -912,9 +908,10 @@ extern "C" int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, 
     return od_launch_status();
   }
   // Two or more chunks: a role per wave (4 x 4096 tokens, 32 heads, both kernels: 508 -> 220 us; 1 x 8192: 887 -> 322;
-  // 2 chunks of 64 sequences: 115 -> 112). Its one workgroup per CU loses to three of the other where two chunks come
-  // with more work than about 16 workgroups per CU (2 chunks of 256 sequences: 385 -> 401).
-  if (nchunk > 2 || (nchunk == 2 && cblocks <= 4096))
+  // 2 chunks of 4 sequences: 15.8 on gdn_chunk_state, 12.4 here). Its one workgroup per CU loses to three of the other
+  // where two chunks come with more than four workgroups per CU (32 heads, 64 tokens, S = 8: 20.4 and 19.0; 16: 30.8
+  // and 31.9; 32: 50 and 56; 256: 319 and 401).
+  if (nchunk > 2 || (nchunk == 2 && cblocks <= 4 * od_cu_count()))
     gdn_chunk_roles_kernel<false><<<dim3((unsigned)cblocks), dim3(64 * (kChain + 4)), 0, (hipStream_t)stream>>>(cp);
   else
     gdn_chunk_state_kernel<<<dim3((unsigned)cblocks), dim3(256), 0, (hipStream_t)stream>>>(cp);

@@ -257,6 +257,46 @@ def test_gdn_chunk_chain_edges(gpu_lib, S, L, n_k, n_v, dv, gmul):
     assert torch.allclose(fs.cpu(), st_r.float(), rtol=1e-5, atol=1e-5 * st_r.abs().max().item())
 
 
+@pytest.mark.parametrize("S,L,final", [(16, 33, True), (16, 64, False), (17, 33, False), (17, 64, True)])
+def test_gdn_two_chunks_over_many_sequences(gpu_lib, S, L, final):
+    """Two chunks on both sides of the line between the two kernels that take them (four blocks of 64 columns
+    per CU: 16 sequences of 32 heads of 128). The first, a middle and the last sequence against float64, with the bars of
+    test_gdn_recurrence_matches_float64, but an absolute floor of 2^-16 of the largest output (a product keeps 16 bits
+    of terms of that size, and among this many outputs some cancel); all of them against the token-by-token kernel, which
+    may be as far off the other way."""
+    from opendecider_amd import kernels
+    n_k, n_v, dv = 16, 32, 128
+    g = torch.Generator().manual_seed(S * 1000 + L)
+    q, k, v, gg, beta = _rec_inputs(g, S, L, n_k, n_v, dv=dv)
+    st0 = torch.randn(2, n_v, 128, dv, generator=g) * 0.5
+    seq = torch.randint(0, 3, (S,), generator=g, dtype=torch.int32)  # 2: outside the states, zeros
+    print(f"gdn two chunks S={S} L={L} final={final}", flush=True)
+    qk = torch.cat([q.reshape(S * L, -1), k.reshape(S * L, -1)], 1)
+    args = [x.to(DEV) for x in (qk, v.reshape(S * L, -1), gg, beta)]
+    kw = dict(init=st0.to(DEV), seq_state=seq.to(DEV), final=final)
+    o, fs = kernels.gdn_recurrence(*args, S, L, n_k, n_v, 128, dv, **kw)
+    o1, fs1 = kernels.gdn_recurrence(*args, S, L, n_k, n_v, 128, dv, chunked=False, **kw)
+    o, o1 = o.cpu().float(), o1.cpu().float()
+    floor = 2.0 ** -16 * o1.abs().max().item()
+    assert ((o - o1).abs() <= o1.abs() * 2.0 ** -6 * 1.01 + 2 * floor).all()
+    rep, pick = n_v // n_k, [0, S // 2, S - 1]
+
+    def rows(x, *shape):
+        return x.reshape(S, L, *shape)[pick]
+
+    init = torch.cat([st0, torch.zeros(1, n_v, 128, dv)])[seq.long()[pick]]
+    o_r, st_r = og.recurrence(rows(q.repeat_interleave(rep, 1), n_v, 128), rows(k.repeat_interleave(rep, 1), n_v, 128),
+                              rows(v, n_v, dv), rows(gg, n_v), rows(beta, n_v), init, torch.float64)
+    o_r = o_r.reshape(len(pick), L, -1).float()
+    d = (rows(o, n_v * dv) - o_r).abs()
+    assert (d <= o_r.abs() * 2.0 ** -7 + floor).all(), d.max().item()
+    assert (d.norm() / o_r.norm()).item() <= 2e-3
+    assert final == (fs is not None)
+    if final:
+        assert torch.allclose(fs.cpu()[pick], st_r.float(), rtol=1e-5, atol=1e-5 * st_r.abs().max().item())
+        assert torch.allclose(fs, fs1, rtol=2e-5, atol=2e-5 * fs1.abs().max().item())
+
+
 @pytest.mark.parametrize("S,L,n_k,n_v,dv,states", [(1, 1, 2, 4, 128, 1), (3, 32, 1, 2, 128, 0), (200, 5, 2, 4, 128, 3),
                                                    (130, 31, 1, 8, 128, 2), (70, 9, 2, 4, 256, 3), (5, 24, 2, 4, 64, 2)])
 def test_gdn_one_chunk_rows(gpu_lib, S, L, n_k, n_v, dv, states):
