@@ -896,13 +896,16 @@ extern "C" int od_gdn_recurrence_chunked(const uint16_t* qk, const uint16_t* v, 
   TArgs tp{qk, g, beta, ws, L, nchunk, (int)n_k, (int)n_v};
   gdn_chunk_t_kernel<<<dim3((unsigned)tblocks), dim3(64), 0, (hipStream_t)stream>>>(tp);
   CArgs cp{qk, v, init, seq_state, ws, o, final_state, L, nchunk, n_states, (int)n_k, (int)n_v, (int)dv, S, 1};
-  // One chunk and no state kept (option rows): runs of sequences that share S_0 in registers, a workgroup per CU (256 x
-  // 24 tokens over 4 states, 32 heads, with T: 227 us on gdn_chunk_state, 75 here; 6 x 24: 17.4 and 12.8). Its eight
-  // chain waves take 128 columns; other widths, and a state that has to be written per sequence (2 MB each, which is
-  // what such a call then takes its time for), stay on gdn_chunk_state.
+  // One chunk and no state kept (option rows): runs of sequences that share S_0 in registers, as few rounds of one
+  // workgroup per CU as kMaxRun allows, of equal runs (rounded down, 15 x 24 tokens of 32 heads took two rounds, 19.8
+  // us, and 300 x 24 141, in place of 15.6 and 95). 256 x 24 tokens, with T: over 4 states 227 us on gdn_chunk_state,
+  // 82 here, over 4 in turn (a state read at every step) 227 and 118, over 256 of their own 256 and 166; 6 x 24: 17.4
+  // and 12.3. Its eight chain waves take 128 columns; other widths, and a state that has to be written per sequence
+  // (2 MB each, which is what such a call then takes its time for), stay on gdn_chunk_state.
   if (nchunk == 1 && !final_state && dv % (16 * kRowChain) == 0) {
     const int64_t heads = n_v * (dv / (16 * kRowChain));
-    cp.run = (int)min((int64_t)kMaxRun, max((int64_t)1, S * heads / 256));
+    const int64_t per = (S * heads + od_cu_count() - 1) / od_cu_count(), rounds = (per + kMaxRun - 1) / kMaxRun;
+    cp.run = (int)((per + rounds - 1) / rounds);
     const int64_t blocks = (S + cp.run - 1) / cp.run * heads;
     gdn_chunk_roles_kernel<true><<<dim3((unsigned)blocks), dim3(64 * (kRowChain + 4)), 0, (hipStream_t)stream>>>(cp);
     return od_launch_status();

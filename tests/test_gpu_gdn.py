@@ -328,6 +328,13 @@ def test_gdn_one_chunk_rows(gpu_lib, S, L, n_k, n_v, dv, states):
     assert (d.norm() / o_r.norm()).item() <= 2e-3
 
 
+@pytest.mark.parametrize("S,L,n_k,n_v", [(9, 3, 16, 32), (15, 2, 16, 32), (4097, 1, 2, 4)])
+def test_gdn_row_runs_are_one_round(gpu_lib, S, L, n_k, n_v):
+    """Row counts that do not fill a round of one workgroup per CU: runs of two with a shorter last one, and more rows
+    than a round of the longest runs takes (two rounds of equal runs)."""
+    test_gdn_one_chunk_rows(gpu_lib, S, L, n_k, n_v, 128, 3)
+
+
 @pytest.mark.parametrize("S,L,n_k,n_v", [(1, 1, 1, 1), (2, 15, 1, 2), (1, 16, 2, 6), (1, 17, 2, 4), (3, 31, 1, 3),
                                          (1, 32, 2, 4), (2, 33, 2, 2), (2, 48, 1, 2)])
 @pytest.mark.parametrize("same_key", [False, True])
