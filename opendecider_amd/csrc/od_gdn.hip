@@ -57,18 +57,10 @@ __device__ __forceinline__ void load16(const uint16_t* p, float (&f)[kChan]) {
   }
 }
 
-__device__ __forceinline__ void store16(uint16_t* p, const float (&f)[kChan]) {
-  uint32_t w[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w[i] = (uint32_t)od_f32_to_bf16(f[2 * i]) | ((uint32_t)od_f32_to_bf16(f[2 * i + 1]) << 16);
-  *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
-  *reinterpret_cast<uint4*>(p + 8) = make_uint4(w[4], w[5], w[6], w[7]);
-}
-
 __device__ __forceinline__ float bf(float x) { return od_bf16_to_f32(od_f32_to_bf16(x)); }
 
-// od_silu_bf16 with its float64 step out of line: the prep kernel calls it for 16 channels per token, and 16
-// inlined copies of the rare float64 path cost registers the common path needs
+// od_silu_bf16 with its float64 step out of line: inlined copies of the rare path would cost registers that the common
+// path needs
 __device__ __noinline__ float silu_bf16_slow(float g) {
   const double gd = (double)g;
   return od_bf16_to_f32(od_f32_to_bf16((float)(gd / (1.0 + exp(-gd)))));
@@ -107,10 +99,12 @@ __device__ __forceinline__ float silu_bf16(float g) {
 //   conv    four float64 fma per channel on taps and a window kept in float64 (one conversion per input; an fp32 chain
 //           with an error bound fails it on 0.3% of channels, the ties of sums of 16-bit products)
 //   silu    of a bf16 value: a 6 KB LDS table of it for 2^-8 <= |g| < 16 and the exponent-decrement of g below (as the
-//           SwiGLU GEMM epilogue has it), in packed 16-bit steps over two channels; lanes with another g call the function
-//   l2norm  fp32 sum S of positive terms, off by at most 11 2^-24 S: bf16(S (1 - 2^-20)) == bf16(S (1 + 2^-20)) proves
-//           its rounding; rsq within 1 ulp, so its bf16 is right unless the low half lies within 4 ulps of the midpoint;
-//           else (1 wave in 200) float64
+//           SwiGLU GEMM epilogue has it), in packed 16-bit steps over two channels; lanes with another g call the
+//           function
+//   l2norm  fp32 sum S of positive terms, NCH / 2 rounded additions in the lane and log2 G across the lanes: with 8
+//           channels at most 4 + 6, off by 10 2^-24 S, with 16 at most 8 + 6, 14 2^-24 S; bf16(S (1 - 2^-20)) ==
+//           bf16(S (1 + 2^-20)), a margin of 16 2^-24 S, proves its rounding; rsq within 1 ulp, so its bf16 is right
+//           unless the low half lies within 4 ulps of the midpoint; else (1 wave in 200) float64
 constexpr int kTok = 16;
 constexpr int kPrepChan = 8;
 constexpr int kPrepThreads = 256;

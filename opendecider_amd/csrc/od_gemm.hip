@@ -879,9 +879,10 @@ struct SplitPlan {
 // Shapes for the small-M kernel (w8a8_gemm_small_kernel): up to 512 rows and at most two of its 64 x 64 tiles per
 // CU (it runs one workgroup per CU and pays each tile's first-chunk latency in full; M = 512 x N = 6144 is faster on
 // the 128 x 256 tiles with split-K). Its tile width, 32, 64 or 96 columns: the one whose rounds of one tile per CU
-// take the least. The 64 rows of A are read whatever the width: one round at K = 4096 measures 8.0, 12.0 and 16.7 us
-// (10.4, 13.9 and 18.5 with W from HBM), 0.67 and 1.33 of the 64-wide one. 192 x 4096 x 12288 in one round of 64 takes
-// 31 us, in two of 32 42; 256 x 6144 x 4096 in one round of 96 18.5, in two of 64 26.
+// take the least. The 64 rows of A are read whatever the width: with W from HBM, as a decoder's layers find it, one
+// round at K = 4096 measures 10.4, 13.9 and 18.5 us, 0.75 and 1.33 of the 64-wide one (8.0, 12.0 and 16.7 with W in the
+// caches: 0.67 and 1.39, which choose alike but for 64 of the shapes). 192 x 4096 x 12288 in one round of 64 takes 31
+// us, in two of 32 42; 256 x 6144 x 4096 in one round of 96 18.5, in two of 64 26.
 constexpr int64_t kSmallMaxM = 512;
 bool small_m(int64_t M, int64_t N) {
   return M <= kSmallMaxM && ((M + kSmBM - 1) / kSmBM) * ((N + 63) / 64) <= 2 * (int64_t)od_cu_count();
@@ -892,7 +893,7 @@ int small_bn(int64_t M, int64_t N) {
   double t = 1e30;
   for (const int bn : {64, 32, 96}) {
     const int64_t rounds = (tm * ((N + bn - 1) / bn) + cus - 1) / cus;
-    const double e = (double)rounds * (bn == 32 ? 0.67 : bn == 64 ? 1.0 : 1.33);
+    const double e = (double)rounds * (bn == 32 ? 0.75 : bn == 64 ? 1.0 : 1.33);
     if (e < t) {
       t = e;
       best = bn;
