@@ -1009,7 +1009,8 @@ __device__ __forceinline__ void branched_attn_body(const AttnArgs& p, Smem<D>& s
       // the int8 state, converted here: registers first, then LDS. A block is loaded right after the block before it is
       // converted, a whole step ahead of its own conversion: issued between the softmax and the P.V product of the
       // same step, the conversion waited for most of the memory latency (8 states x 32768 keys, 128 slots per head: 271
-      // -> 256 us; bound now by its 587 vector instructions per block and wave, half of them the conversion)
+      // -> 256 us; now 587 vector instructions, half of them the conversion, and 32 MFMAs per block and wave, at most 59%
+      // and 26% of the cycles)
       const PrefixSrc src = prefix_src<D>(p.kq, p.ks, p.vq, p.vs, p.kvalid, p.Hkv, p.T, p.cap, s, g);
       PrefixRegs<D> pr;
       prefix_load<D>(src, p.T, b_lo * kBlockKeys, pr);

@@ -632,7 +632,8 @@ def branched_attn(q, k_own, v_own, kq, ks, vq, vs, scale: float, kvalid=None, ro
     kq/vq (Ns, Hkv, cap, D) int8 of which the first T tokens are used (T = `length`, else kvalid.shape[1], else
     cap); ks/vs (Ns, Hkv, cap) fp32; kvalid (Ns, T) bool/uint8 or None.
     Rows are grouped by state: row_counts (host ints, one per state) or a prebuilt (row_start, max_rows) pair from
-    row_start_of(); neither means Ns == 1. n_split: key-range splits; None picks them from the grid size
+    row_start_of() (ordered on the stream that built it, unless kept); neither means Ns == 1. n_split: key-range
+    splits; None picks them from the grid size
     (split_count). staged: convert the state once into block images (od_attn_stage, into `stage_buf` when given and
     large enough) and run od_branched_attn_staged over them; False runs od_branched_attn / od_branched_attn_split,
     which convert in every workgroup (same results, bit for bit); None stages when at least STAGE_MIN_TILES slot
