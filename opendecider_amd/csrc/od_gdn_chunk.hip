@@ -520,7 +520,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_state_kernel(CArgs p) {
 //                       stores of chunk c - 1
 // Each role is a loop of its own (the registers of one role are not live in the other) with one barrier per chunk
 // over three stage buffers. Bound: the chain wave's own chunk, ~210 vector instructions, 64 MFMAs and ~45 LDS reads in
-// sequence, about 2500 cycles, with the staging waves just below it (4 x 4096 tokens, 32 heads: 2950 cycles a chunk
+// sequence, about 2500 cycles, with the staging waves just below it (4 x 4096 tokens, 32 heads: 2900 cycles a chunk
 // against 6500 with every wave doing all of it, 476 -> 175 us; one workgroup per CU, LDS 110 KB).
 // Rows of K, Q, V, T and P are staged in the order row(j) = 16 ((j >> 2) & 1) + 4 (j >> 3) + (j & 3) and the state's dk
 // rows alike within each 32, which makes accumulator tiles 0 and 1 of a lane group h hold tokens (dk) 8 h .. 8 h + 7 in

@@ -326,7 +326,7 @@ def test_two_level_without_questions_equals_one_level(gpu_lib):
 
 @pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 1400])
 def test_row_offsets_without_a_copy(gpu_lib, n):
-    """row_start_of's device offsets (kernel arguments, 512 per launch) are the running sums, also behind other work on
+    """row_start_of's device offsets (up to 512 kernel arguments, more by a copy, in a graph 512 per launch) are the sums, also behind other work on
     a side stream and inside a captured graph."""
     from opendecider_amd import kernels
     counts = [(7 * i) % 5 for i in range(n)]

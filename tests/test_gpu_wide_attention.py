@@ -165,8 +165,8 @@ def test_scale_must_be_positive():
 def test_left_pads_and_stream_order(gpu_lib, B, H, G, T, S, DK, DV, pads, causal):
     """Left-padded states, whose leading blocks are skipped: pads of no, whole and partial 64-key blocks, past the first
     1024 keys scanned, over every key (outputs 0, LSE -inf) and over every key that early queries see; on the LDS-DMA
-    path with and without halves and on the register-staged path; (batch, group) counts that are not multiples of 8
-    (tiles of all streams side by side), with 1 and 2 halves."""
+    path with and without halves and on the register-staged path; (batch, group) counts that are not multiples of 8,
+    with 1 and 2 halves."""
     q, k, v, _ = make(B * 100 + S + DK, B, H, G, T, S, DK, DV, False)
     kv = torch.arange(S)[None, :] >= torch.tensor(pads)[:, None]
     out, lse = run(q, k, v, kv, causal)
